@@ -8,10 +8,11 @@
 //     terms -- one elementwise pass;
 //   propagators as the reference's q_s = e^{-W_b(s)} F^-1[g F q_{s-1}]
 //     (fts_molecule_linear.cu:144-269), D = F^-1 g F applied axis by axis
-//     because g(k) = exp(-k^2/(Nr-1)) factorises over kx, ky, kz: the x-y pass
-//     reads q_{s-1} alone and the z pass multiplies by E_b(s), so a bead costs
-//     two reads and two writes of a slice plus one read of E; the forward and
-//     complementary chains of every replica share each launch;
+//     because g(k) = exp(-k^2/(Nr-1)) factorises over kx, ky, kz: one launch a
+//     bead with the axes as real matrices (fts_bead.h) where every length is one
+//     of its, else an x-y pass that reads q_{s-1} alone and a z pass that
+//     multiplies by E_b(s); the forward and complementary chains of every
+//     replica share each launch;
 //   density: rho_b ~ e^{W_b} sum_s q_s qdag_{N-1-s} (fts_molecule_linear.cu:
 //     298-327) and Q = gvol/V sum q_{N-1}, FP64 accumulation; the n/(QV)
 //     factor is applied by the next update.
@@ -28,8 +29,16 @@
 
 #include "common.h"
 #include "fft_core.h"
+#include "fts_bead.h"
 
 namespace mft {
+
+// fts_bead.hip
+bool bead_length(int n);
+void bead_table(int n, const double* g, std::vector<float>& tab);
+int bead_allow_lds(int nx, int na);
+int bead_launch(const BeadDesc* h, const BeadDesc* d, int n, const int dims[3], int axis, hipStream_t st);
+
 
 const float2* fft_twiddles_device(int n); // fft.hip
 
@@ -762,6 +771,7 @@ struct FtsRep {
     float2 *p[kFtsMaxMol] = {nullptr}, *pd[kFtsMaxMol] = {nullptr};
     float2* tmp = nullptr; // [2*nmol][M]
     float2* g[3] = {nullptr, nullptr, nullptr};
+    float* bt[3] = {nullptr, nullptr, nullptr}; // bead_table() per axis (grids of the bead kernel)
     double *Hpart = nullptr, *Qpart = nullptr;
     double2* Q = nullptr;
     int nHpart = 0, nQpart = 0;
@@ -794,6 +804,12 @@ struct FtsGroup {
     // (1..maxN-1) and axis a descriptor list
     std::vector<std::vector<PropDesc*>> d_prop;   // [chunk][step*3 + axis]
     std::vector<std::vector<int>> nprop;          // [chunk][step] chains
+    // grids the bead kernel covers: per chunk and step s (0 starts bead 1) the
+    // first descriptor and the number of chains
+    bool bead = false;
+    std::vector<BeadDesc> h_bead;
+    BeadDesc* d_bead = nullptr;
+    std::vector<std::vector<std::pair<size_t, int>>> bead_at;
     size_t chunk_bytes = 0;
     int maxN = 0;
     bool dirty = false;              // membership changed: rebuild descriptors
@@ -894,14 +910,20 @@ static int validate_desc(const mft_fts_desc& d)
     return MFT_OK;
 }
 
-// exp(-k^2/(Nr-1))/n per axis as an unevaluated float sum hi + lo; k from
-// the reference's float wavevector (Box.cu:182-203)
+// exp(-k^2/(Nr-1)) of one axis; k from the reference's float wavevector
+// (Box.cu:182-203)
+static double axis_factor(int i, int n, float L, double Nr)
+{
+    const double k = (double)kcomp(i, n, L);
+    return std::exp(-k * k / (Nr - 1.0));
+}
+
+// the same over n as an unevaluated float sum hi + lo
 static void axis_table(int n, float L, double Nr, std::vector<float2>& g)
 {
     g.resize(n);
     for (int i = 0; i < n; ++i) {
-        double k = (double)kcomp(i, n, L);
-        double v = std::exp(-k * k / (Nr - 1.0)) / (double)n;
+        double v = axis_factor(i, n, L, Nr) / (double)n;
         float hi = (float)v;
         g[i] = make_float2(hi, (float)(v - (double)hi));
     }
@@ -993,6 +1015,9 @@ static int linear_coeffs(FtsRep& r)
     return MFT_OK;
 }
 
+// whether a grid's chains are propagated by the bead kernel
+static bool bead_grid(const int n[3]) { return bead_length(n[0]) && bead_length(n[1]) && bead_length(n[2]); }
+
 static int rep_setup(FtsBatch* b, FtsRep& r)
 {
     const mft_fts_desc& d = r.d;
@@ -1066,6 +1091,18 @@ static int rep_setup(FtsBatch* b, FtsRep& r)
         axis_table(ns[a], Ls[a], d.Nr, g);
         if ((rc = dev_alloc(r.allocs, &r.g[a], g.size()))) return rc;
         MFT_HIP(hipMemcpy(r.g[a], g.data(), sizeof(float2) * g.size(), hipMemcpyHostToDevice));
+    }
+    if (b->plane_xy && bead_grid(ns)) {
+        for (int a = 0; a < 3; ++a) {
+            std::vector<double> g(ns[a]);
+            for (int i = 0; i < ns[a]; ++i) g[i] = axis_factor(i, ns[a], Ls[a], d.Nr);
+            std::vector<float> tab;
+            bead_table(ns[a], g.data(), tab);
+            if ((rc = dev_alloc(r.allocs, &r.bt[a], tab.size()))) return rc;
+            MFT_HIP(hipMemcpy(r.bt[a], tab.data(), sizeof(float) * tab.size(), hipMemcpyHostToDevice));
+        }
+        for (int a = 1; a < 3; ++a)
+            if ((rc = bead_allow_lds(ns[0], ns[a]))) return rc;
     }
     r.nHpart = (r.M + kFtsThreads - 1) / kFtsThreads;
     r.nQpart = r.nHpart;
@@ -1172,6 +1209,47 @@ static int bead_species(const mft_fts_molecule& mol, int Ntot, int s, int c)
     return mol.species[mol.nblocks - 1];
 }
 
+// descriptors of the bead kernel, uploaded at once: step 0 starts bead 1 from
+// q_0 along y, step s finishes bead s along z (odd s) or y (even s) and starts
+// the next
+static int group_beads(FtsBatch* b, FtsGroup& G, const std::vector<int>& chunk_end)
+{
+    std::vector<BeadDesc>& all = G.h_bead;
+    all.clear();
+    for (size_t ch = 0; ch < chunk_end.size(); ++ch) {
+        G.bead_at.emplace_back();
+        for (int s = 0; s < G.maxN; ++s) {
+            const size_t first = all.size();
+            for (int k = ch == 0 ? 0 : chunk_end[ch - 1]; k < chunk_end[ch]; ++k) {
+                FtsRep& r = b->reps[G.reps[k]];
+                int chain = 0;
+                for (int m = 0; m < r.d.nmolecules; ++m)
+                    for (int c = 0; c < (r.sym[m] ? 1 : 2); ++c, ++chain) {
+                        const int last = r.Ntot[m] - 1;
+                        if (s > last || last == 0) continue;
+                        float2* P = c == 0 ? r.p[m] : r.pd[m];
+                        float2* tmp = r.tmp + (size_t)chain * r.M;
+                        BeadDesc D;
+                        D.src = s == 0 ? P : tmp;
+                        D.dst = s < last ? tmp : nullptr;
+                        D.E = s == 0 ? nullptr
+                                     : r.E + (size_t)bead_species(r.d.molecules[m], r.Ntot[m], s, c) * r.M;
+                        D.q = P + (size_t)s * r.M;
+                        D.ta = r.bt[s & 1 ? 2 : 1];
+                        D.tx = r.bt[0];
+                        all.push_back(D);
+                    }
+            }
+            G.bead_at[ch].push_back({first, (int)(all.size() - first)});
+        }
+    }
+    int rc;
+    if ((rc = dev_alloc(G.allocs, &G.d_bead, all.size()))) return rc;
+    if (!all.empty())
+        MFT_HIP(hipMemcpy(G.d_bead, all.data(), sizeof(BeadDesc) * all.size(), hipMemcpyHostToDevice));
+    return MFT_OK;
+}
+
 static int group_setup(FtsBatch* b, FtsGroup& G)
 {
     int rc;
@@ -1276,6 +1354,9 @@ static int group_setup(FtsBatch* b, FtsGroup& G)
     }
     chunk_end.push_back(nr);
     const int nchunks = (int)chunk_end.size();
+    G.bead = b->plane_xy && bead_grid(G.n);
+    G.bead_at.clear();
+    if (G.bead) return group_beads(b, G, chunk_end);
     G.d_prop.assign(nchunks, std::vector<PropDesc*>((size_t)3 * G.maxN, nullptr));
     G.nprop.assign(nchunks, std::vector<int>(G.maxN, 0));
     for (int ch = 0; ch < nchunks; ++ch)
@@ -1332,7 +1413,8 @@ static int launch_prop(const PropDesc* d, int n, const FtsGroup& G, int axis, hi
     return MFT_OK;
 }
 
-// whether the x and y passes of this group run as one plane kernel
+// whether the x and y passes of this group run as one plane kernel (grids with
+// such planes whose third length the bead kernel does not take)
 static bool plane_fused(const FtsGroup& G)
 {
     if (G.n[0] != G.n[1]) return false;
@@ -1379,6 +1461,11 @@ static int group_density(FtsBatch* b, FtsGroup& G)
     int rc;
     hipStream_t st = b->stream;
     const bool fused = plane_fused(G) && b->plane_xy;
+    for (const auto& chunk : G.bead_at)
+        for (int s = 0; s < (int)chunk.size(); ++s)
+            if (chunk[s].second > 0 &&
+                (rc = bead_launch(G.h_bead.data() + chunk[s].first, G.d_bead + chunk[s].first, chunk[s].second, G.n, s & 1 ? 2 : 1, st)))
+                return rc;
     for (size_t ch = 0; ch < G.d_prop.size(); ++ch) {
         const std::vector<PropDesc*>& dp = G.d_prop[ch];
         for (int s = 1; s < G.maxN; ++s) {
@@ -1492,8 +1579,8 @@ static FtsGroup& group_for(FtsBatch* b, const FtsRep& r)
 static int batch_create_empty(FtsBatch** out, int nslots)
 {
     FtsBatch* b = new FtsBatch();
-    // MFT_FTS_PLANE_XY=0 keeps the x and y passes as separate line kernels
-    // (same arithmetic; used to check that the plane kernel matches them)
+    // MFT_FTS_PLANE_XY=0 keeps every axis a pass of line transforms (to check
+    // that the bead kernel and the plane kernel match them)
     const char* pe = std::getenv("MFT_FTS_PLANE_XY");
     b->plane_xy = !(pe && pe[0] == '0');
     // MFT_FTS_GRAPH=0 launches every iteration directly (checks the replayed
