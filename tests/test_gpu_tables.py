@@ -1,0 +1,71 @@
+"""Table kernels and the pair force of the per-kernel entry points where their
+work split has edges: particle counts around a workgroup's share, every spline
+order, table rows that are no multiple of the lanes that share them, site lists
+with entries out of range, and grids down to two points with a k-space table of
+no symmetry.
+
+Tolerances: a mapped force adds G <= 125 products in float, at most G + 8
+roundings of 2^-24 relative to the sum of their magnitudes; the pair force is
+three float transforms of at most log2(M) <= 16 levels each way, 4 roundings of
+2^-24 a level and an rms growth of its square root, within 2e-6 normwise.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+
+import orc
+from test_gpu_fts import rel, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("p", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("ns", [1, 31, 32, 33, 257])
+def test_tables_around_a_workgroups_share(gpu, p, ns):
+    rng = np.random.default_rng(100 * p + ns)
+    Nx, L = (12, 10, 16), np.array([4.0, 3.0, 5.0], np.float32)
+    dx = (L / np.array(Nx, np.float32)).astype(np.float32)
+    x = (rng.random((ns, 3)) * L).astype(np.float32).reshape(-1)
+    G, M, gvol = (p + 1) ** 3, int(np.prod(Nx)), float(np.prod(dx.astype(np.float64)))
+    inds, W = gpu.grid_weights(x, Nx, dx, p)
+    inds_o, W_o = orc.grid_weights(x, Nx, dx, p)
+    assert np.array_equal(inds, inds_o)
+    assert rel(W, W_o) < 1e-6  # three weights, a product and a division
+    # a group of every second particle, with sites that are no particles
+    sites = np.concatenate([np.arange(0, ns, 2), [-1, ns, ns + 7]]).astype(np.int32)
+    q = rng.normal(size=ns).astype(np.float32)
+    Wd = W.astype(np.float64).reshape(ns, G)
+    rho, rhoq = gpu.fill_density(M, sites, inds, W, G, q=q)
+    own = np.arange(0, ns, 2)
+    want, wantq = np.zeros(M), np.zeros(M)
+    np.add.at(want, inds.reshape(ns, G)[own], Wd[own])
+    np.add.at(wantq, inds.reshape(ns, G)[own], Wd[own] * q[own, None])
+    # fixed point of 2^-32 a product, one rounding of the sum
+    lim = len(own) * G * 2.0 ** -33
+    assert np.max(np.abs(rho - want)) <= lim + 2.0 ** -24 * np.max(np.abs(want))
+    assert np.max(np.abs(rhoq - wantq)) <= lim + 2.0 ** -23 * np.max(np.abs(Wd)) * 4 * len(own)
+    F = rng.normal(size=(M, 3)).astype(np.float32)
+    f = gpu.map_forces(ns, F.reshape(-1), sites, inds, W, G, gvol, q=q).reshape(ns, 3)
+    terms = F.astype(np.float64)[inds.reshape(ns, G)] * (Wd * gvol)[:, :, None]
+    want = terms.sum(1) * q[:, None]
+    bound = (G + 8) * 2.0 ** -24 * np.abs(terms).sum(1) * np.abs(q)[:, None]
+    assert np.all(np.abs(f - want)[own] <= bound[own])
+    assert not f[np.setdiff1d(np.arange(ns), own)].any()
+
+
+@pytest.mark.parametrize("grid", [(2, 3, 5), (16, 2, 4), (12, 20, 24), (40, 6, 48), (64, 10, 3), (8, 64, 80)])
+def test_pair_force_of_a_table_without_symmetry(gpu, grid):
+    rng = np.random.default_rng(sum(grid))
+    M = int(np.prod(grid))
+    rho = rng.normal(size=M).astype(np.float32)
+    fk = (rng.normal(size=(M, 3)) + 1j * rng.normal(size=(M, 3))).astype(np.complex64)
+    F0 = rng.normal(size=(M, 3)).astype(np.float32)
+    got = gpu.pair_force(F0.reshape(-1), rho, fk, grid, factor=1.7).reshape(M, 3)
+    sh = grid[::-1]
+    S = np.fft.fftn(rho.reshape(sh).astype(np.float64)) / M
+    for j in range(3):
+        V = np.fft.ifftn(fk[:, j].reshape(sh) * S) * M
+        e = rel(got[:, j], F0[:, j] + 1.7 * V.real.reshape(-1))
+        say("pair force", grid, j, "%.2e" % e)
+        assert e < 2e-6
