@@ -272,7 +272,7 @@ struct TildEngine {
     // binning
     TileGeom tg;
     int nkeys = 0;
-    int *count = nullptr, *start = nullptr, *partial = nullptr;
+    int *count = nullptr, *start = nullptr, *partial = nullptr; // count: two buffers (slot_count)
     int nscan_blocks = 0;
     // grids
     float* rho = nullptr;   // [nchan][M], reduced from the tiles when read
@@ -334,6 +334,9 @@ struct TildEngine {
 // every bond is then type 0 (set_topology checks the range), so the slots'
 // types are neither carried through the permutation nor read.
 inline int* slot_bond_types(const TildEngine* e, int c) { return e->bp.ntypes > 1 ? e->BT[c] : nullptr; }
+
+// key counts of the step that starts from buffer c
+inline int* slot_count(const TildEngine* e, int c) { return e->count + (size_t)c * e->nkeys; }
 
 constexpr int kBlock = 256;
 inline unsigned nblk(long n) { return (unsigned)((n + kBlock - 1) / kBlock); }

@@ -330,26 +330,31 @@ __global__ void k_scan_reduce(const int* __restrict__ count, int M, int* __restr
     if (threadIdx.x == 0) partial[blockIdx.x] = tot;
 }
 
-// start[i] = exclusive prefix of count; count cleared for the next binning.
-// Each block adds the totals of the blocks before it (at most a few thousand
-// values, read from L2), so the scan takes two launches.
-__global__ void k_scan_apply(int* __restrict__ count, int M, const int* __restrict__ partial,
-                             int* __restrict__ start, int ns, uint32_t* __restrict__ dstep)
+// Keys a thread of the scan takes: 16, as four int4 loads and stores (the number
+// of keys is a multiple of 64, the sub-cells of a brick and species, so a thread's
+// keys are all in range or all past it).
+static_assert(kScanItems == 16, "four int4 per thread");
+
+// start[i] = exclusive prefix of count.  The counts come in two buffers that
+// alternate between steps: `other`, read by the previous step's scan, is cleared
+// here for the next one.  Each block adds the totals of the blocks before it (at
+// most a few thousand values, read from L2); one block needs none.
+__global__ void k_scan_apply(const int* __restrict__ count, int* __restrict__ other, int M,
+                             const int* __restrict__ partial, int* __restrict__ start, int ns,
+                             uint32_t* __restrict__ dstep)
 {
     __shared__ int sh[16];
+    const long first = (long)blockIdx.x * blockDim.x * kScanItems;
     int c = 0;
     for (int j = threadIdx.x; j < (int)blockIdx.x; j += blockDim.x) c += partial[j];
-    int carry;
-    block_exclusive_scan(c, sh, &carry);
-    // M is a multiple of 64 (64 sub-cell keys per brick and species), so a
-    // thread's 16 keys are all in range or all past it: int4 loads and stores
-    static_assert(kScanItems == 16, "four int4 per thread");
-    const long base = (long)blockIdx.x * kScanChunk + (long)threadIdx.x * kScanItems;
+    const long base = first + (long)threadIdx.x * kScanItems;
     const bool in = base < M;
     int4 v4[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k)
         v4[k] = in ? reinterpret_cast<const int4*>(count + base)[k] : make_int4(0, 0, 0, 0);
+    int carry;
+    block_exclusive_scan(c, sh, &carry);
     int s = 0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) s += v4[k].x + v4[k].y + v4[k].z + v4[k].w;
@@ -365,7 +370,7 @@ __global__ void k_scan_apply(int* __restrict__ count, int M, const int* __restri
             o.w = o.z + v4[k].z;
             ex = o.w + v4[k].w;
             reinterpret_cast<int4*>(start + base)[k] = o;
-            reinterpret_cast<int4*>(count + base)[k] = make_int4(0, 0, 0, 0);
+            reinterpret_cast<int4*>(other + base)[k] = make_int4(0, 0, 0, 0);
         }
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -1666,11 +1671,11 @@ int tild_tiles_configure(TildEngine* e)
     for (void* pbuf : {(void*)e->count, (void*)e->start, (void*)e->partial})
         if (pbuf) (void)hipFree(pbuf);
     e->count = e->start = e->partial = nullptr;
-    if ((rc = dalloc(&e->count, (size_t)e->nkeys))) return rc;
+    if ((rc = dalloc(&e->count, 2 * (size_t)e->nkeys))) return rc;
     if ((rc = dalloc(&e->start, (size_t)e->nkeys + 1))) return rc;
     e->nscan_blocks = (e->nkeys + kScanChunk - 1) / kScanChunk;
     if ((rc = dalloc(&e->partial, (size_t)e->nscan_blocks))) return rc;
-    MFT_HIP(hipMemset(e->count, 0, sizeof(int) * (size_t)e->nkeys));
+    MFT_HIP(hipMemset(e->count, 0, 2 * sizeof(int) * (size_t)e->nkeys));
     e->have_state = 0; // the key order changed: the state is sorted again when set
     return MFT_OK;
 }
@@ -1682,12 +1687,15 @@ int tild_sort_state(TildEngine* e)
     const mft_tild_desc& d = e->d;
     const int N = e->N, mb = std::max(1, d.maxbonds), c = e->cur;
     e->nz_keyed = false; // NZ holds the given previous noise
-    MFT_HIP(hipMemsetAsync(e->count, 0, sizeof(int) * (size_t)e->nkeys, e->stream));
-    k_sort_count<<<nblk(N), kBlock, 0, e->stream>>>(e->pio, e->type, N, e->count, e->key, e->rank, e->dx[0],
+    int* count = slot_count(e, c);
+    MFT_HIP(hipMemsetAsync(count, 0, sizeof(int) * (size_t)e->nkeys, e->stream));
+    k_sort_count<<<nblk(N), kBlock, 0, e->stream>>>(e->pio, e->type, N, count, e->key, e->rank, e->dx[0],
                                                      e->dx[1], e->dx[2], d.pmeorder, d.nx, d.ny, d.nz, e->tg);
     MFT_LAUNCH_CHECK();
     int rc;
     if ((rc = tild_scan(e))) return rc;
+    // the sort stays in this buffer, so the first step counts into it again
+    MFT_HIP(hipMemsetAsync(count, 0, sizeof(int) * (size_t)e->nkeys, e->stream));
     k_sort_place<<<nblk(N), kBlock, 0, e->stream>>>(e->pio, e->pio2, e->pio3, e->charge, e->type,
                                                      e->bondType, mb, N, e->key, e->rank, e->start, e->slot_of,
                                                      e->X[c], e->XO[c], e->NZ[c], e->META[c], e->BT[c]);
@@ -1736,9 +1744,15 @@ int tild_unsort(TildEngine* e, int what)
 int tild_scan(TildEngine* e, bool advance_step)
 {
     uint32_t* ds = (advance_step && e->use_dstep) ? e->d_step : nullptr;
-    k_scan_reduce<<<e->nscan_blocks, kScanThreads, 0, e->stream>>>(e->count, e->nkeys, e->partial);
-    k_scan_apply<<<e->nscan_blocks, kScanThreads, 0, e->stream>>>(e->count, e->nkeys, e->partial, e->start, e->N,
-                                                                    ds);
+    int *count = slot_count(e, e->cur), *other = slot_count(e, 1 - e->cur);
+    // what one block of 1024 threads holds is scanned by it alone (8192 keys:
+    // 5.4 + 3.7 -> 4.9 us); several such blocks that each read the counts before
+    // their own were slower than the reduction's launch (98 304 keys: 13.2 us
+    // against 6.1 + 4.4)
+    const bool one = e->nkeys <= 1024 * kScanItems;
+    if (!one) k_scan_reduce<<<e->nscan_blocks, kScanThreads, 0, e->stream>>>(count, e->nkeys, e->partial);
+    k_scan_apply<<<one ? 1 : e->nscan_blocks, one ? 1024 : kScanThreads, 0, e->stream>>>(
+        count, other, e->nkeys, e->partial, e->start, e->N, ds);
     MFT_LAUNCH_CHECK();
     return MFT_OK;
 }
@@ -1977,14 +1991,15 @@ int tild_integrate(TildEngine* e, bool want_f)
         k_integrate<true><<<nblk(e->N), kBlock, 0, e->stream>>>(e->X[c], e->META[c], e->BS[c],
                                                               slot_bond_types(e, c), e->fgrid,
                                                               want_f ? e->ftot : nullptr, 2, e->bp,
-                                                              step_args(e), e->N, e->count, e->key, e->rank, e->tg,
+                                                              step_args(e), e->N, slot_count(e, c), e->key, e->rank,
+                                                              e->tg,
                                                               ds);
     else
         k_integrate<false><<<nblk(e->N), kBlock, 0, e->stream>>>(e->X[c], e->META[c], e->BS[c],
                                                                slot_bond_types(e, c), e->fgrid,
                                                                want_f ? e->ftot : nullptr,
                                                                std::max(1, d.maxbonds), e->bp, step_args(e), e->N,
-                                                               e->count, e->key, e->rank, e->tg, ds);
+                                                               slot_count(e, c), e->key, e->rank, e->tg, ds);
     MFT_LAUNCH_CHECK();
     return MFT_OK;
 }
