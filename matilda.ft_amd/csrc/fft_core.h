@@ -14,6 +14,7 @@
 // the supported table below.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <type_traits>
 
 namespace mft {
 
@@ -155,7 +156,7 @@ MFT_PLAN(192, 16, 4, 4, 4, 3)
 MFT_PLAN(256, 32, 8, 8, 4)
 #undef MFT_PLAN
 
-// Plans with four elements per thread for kernels that keep several lines
+// Plans with four to ten elements per thread for kernels that keep several lines
 // in registers at once (the fused k-space pass): more threads per line,
 // fewer registers per thread, one more LDS pass.  Sizes without one use the
 // default plan.
@@ -169,11 +170,26 @@ struct FftPlanLow : FftPlan<N> {};
         static constexpr int E = N_ / T_;                                       \
         using R = Radices<__VA_ARGS__>;                                         \
     };
+MFT_PLAN_LOW(16, 4, 4, 4)
+MFT_PLAN_LOW(20, 2, 2, 2, 5)
+MFT_PLAN_LOW(24, 4, 2, 2, 2, 3)
 MFT_PLAN_LOW(32, 8, 4, 4, 2)
+MFT_PLAN_LOW(40, 4, 2, 2, 2, 5)
+MFT_PLAN_LOW(48, 8, 2, 2, 2, 2, 3)
 MFT_PLAN_LOW(64, 16, 4, 4, 4)
+MFT_PLAN_LOW(80, 8, 2, 2, 2, 2, 5)
+MFT_PLAN_LOW(96, 16, 2, 2, 2, 2, 2, 3)
 MFT_PLAN_LOW(128, 32, 4, 4, 4, 2)
+MFT_PLAN_LOW(160, 16, 2, 2, 2, 2, 2, 5)
 MFT_PLAN_LOW(256, 64, 4, 4, 4, 4)
 #undef MFT_PLAN_LOW
+
+// Plans of the particle-mesh engine's x and y passes: the default but where it
+// holds 12 or 20 elements a thread, which serialises a line over two or four
+// threads (24^3, two channels: x pass from the density tiles
+// 11.5 -> 6.5 us, last inverse x pass 7.8 -> 5.4 us).
+template <int N>
+struct FftPlanMesh : std::conditional_t<(FftPlan<N>::E > 8 && N > 12), FftPlanLow<N>, FftPlan<N>> {};
 
 // Expands F(N) for every supported size; used by host dispatch switches.
 #define MFT_FOR_EACH_FFT_SIZE(F)                                                 \
@@ -292,11 +308,12 @@ __device__ __forceinline__ void line_fft(float2 (&v)[N / FftPlan<N>::T], float2*
 }
 
 // The same transform with an explicit plan.
-template <typename Plan, int SIGN>
+template <typename Plan, int SIGN, bool WAVE = false>
 __device__ __forceinline__ void line_fft_plan(float2 (&v)[Plan::E], float2* lds, const float2* tw, int t,
                                               const LdsMap& map)
 {
-    fft_run<Plan::N, Plan::T, SIGN>(v, lds, tw, t, map, typename Plan::R{});
+    static_assert(!WAVE || (Plan::T <= 64 && 64 % Plan::T == 0), "a line must fit in one wavefront");
+    fft_run<Plan::N, Plan::T, SIGN, WAVE>(v, lds, tw, t, map, typename Plan::R{});
 }
 
 // Geometry of the lines along one axis of an x-fastest (nx, ny, nz) grid.

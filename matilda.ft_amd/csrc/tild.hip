@@ -390,7 +390,7 @@ static int grid_forces(TildEngine* e)
                 return rc;
         }
         TimedScope ts(e, MFT_TK_FFT_Y_FWD);
-        if ((rc = tild_axis(-1, 0, 0, e->S, e->S, gy, e->nchan, M, 1.0f, e->stream))) return rc;
+        if ((rc = tild_axis_mesh(-1, e->S, gy, e->nchan, M, e->stream))) return rc;
     }
     {
         TimedScope ts(e, MFT_TK_CONV_Z);
@@ -398,7 +398,7 @@ static int grid_forces(TildEngine* e)
     }
     if (!plane) {
         TimedScope ts(e, MFT_TK_FFT_Y_INV);
-        if ((rc = tild_axis(+1, 0, 0, e->Y, e->Y, gy, e->npk, M, 1.0f, e->stream))) return rc;
+        if ((rc = tild_axis_mesh(+1, e->Y, gy, e->npk, M, e->stream))) return rc;
     }
     {
         TimedScope ts(e, MFT_TK_FFT_X_INV);

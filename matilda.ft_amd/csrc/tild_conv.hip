@@ -16,18 +16,18 @@ __device__ __forceinline__ float pot_shape(const KPot& P, float k2, long idx)
 
 // Fused z pass: forward z FFT of every density channel (already transformed
 // along x and y), k-space forces, inverse z FFT of each output component.
-template <int N, int NCH>
+template <int N, int NCH, int NT>
 __device__ __forceinline__ void conv_z_body(const float2* __restrict__ S, float2* __restrict__ Y, int nx, int ny,
                                             float Lx, float Ly, float Lz, const KParams& kp,
                                             const float2* __restrict__ twg, float invM, double* __restrict__ epart,
                                             float Mgvol)
 {
     using P = FftPlanLow<N>;
-    constexpr int T = P::T, E = P::E, B = 256 / T;
+    constexpr int T = P::T, E = P::E, B = NT / T;
     __shared__ float2 lds[B * N];
     __shared__ float2 tw[N];
-    __shared__ double ered[4 * (kMaxPots + 1)];
-    for (int i = threadIdx.x; i < N; i += 256) tw[i] = twg[i];
+    __shared__ double ered[NT / 64 * (kMaxPots + 1)];
+    for (int i = threadIdx.x; i < N; i += NT) tw[i] = twg[i];
     const int lline = threadIdx.x % B;
     const int t = threadIdx.x / B;
     // consecutive line groups on one XCD: a group's B lines are half of a
@@ -232,7 +232,7 @@ __device__ __forceinline__ void conv_z_body(const float2* __restrict__ S, float2
         __syncthreads();
         if (threadIdx.x < kp.npots) {
             double s = 0.0;
-            for (int w = 0; w < 4; ++w) s += ered[w * (kMaxPots + 1) + threadIdx.x];
+            for (int w = 0; w < NT / 64; ++w) s += ered[w * (kMaxPots + 1) + threadIdx.x];
             epart[(long)blockIdx.x * kMaxPots + threadIdx.x] = s * (double)Mgvol;
         }
     }
@@ -240,21 +240,21 @@ __device__ __forceinline__ void conv_z_body(const float2* __restrict__ S, float2
 
 // Up to three channels the pass fits 128 registers (four waves per SIMD);
 // more channels keep the register count they need.
-template <int N, int NCH>
-__global__ void __launch_bounds__(256, 4) k_conv_z(const float2* __restrict__ S, float2* __restrict__ Y, int nx, int ny,
+template <int N, int NCH, int NT>
+__global__ void __launch_bounds__(NT, 4) k_conv_z(const float2* __restrict__ S, float2* __restrict__ Y, int nx, int ny,
                                                 float Lx, float Ly, float Lz, KParams kp, const float2* __restrict__ twg,
                                                 float invM, double* __restrict__ epart, float Mgvol)
 {
-    conv_z_body<N, NCH>(S, Y, nx, ny, Lx, Ly, Lz, kp, twg, invM, epart, Mgvol);
+    conv_z_body<N, NCH, NT>(S, Y, nx, ny, Lx, Ly, Lz, kp, twg, invM, epart, Mgvol);
 }
 
-template <int N, int NCH>
-__global__ void __launch_bounds__(256) k_conv_z_wide(const float2* __restrict__ S, float2* __restrict__ Y, int nx,
+template <int N, int NCH, int NT>
+__global__ void __launch_bounds__(NT) k_conv_z_wide(const float2* __restrict__ S, float2* __restrict__ Y, int nx,
                                                      int ny, float Lx, float Ly, float Lz, KParams kp,
                                                      const float2* __restrict__ twg, float invM,
                                                      double* __restrict__ epart, float Mgvol)
 {
-    conv_z_body<N, NCH>(S, Y, nx, ny, Lx, Ly, Lz, kp, twg, invM, epart, Mgvol);
+    conv_z_body<N, NCH, NT>(S, Y, nx, ny, Lx, Ly, Lz, kp, twg, invM, epart, Mgvol);
 }
 
 __global__ void k_energy_sum(double* __restrict__ out, const double* __restrict__ part, int nblocks, int npots)
@@ -269,13 +269,24 @@ __global__ void k_energy_sum(double* __restrict__ out, const double* __restrict_
     if (threadIdx.x == 0) out[p] = red[0] + red[1] + red[2] + red[3];
 }
 
+// Threads of a workgroup: one wavefront where 256-thread workgroups would leave
+// compute units idle; the lines then spread over four times the units and their
+// exchanges need no barrier across wavefronts (two channels, with the low plans of
+// 24 and 40 points: 24^3 17.0 -> 10.1 us, 32^3 9.3 -> 7.7, 96 x 64 x 40 26 -> 15.8;
+// from 256 workgroups on, as at 64^3, every unit has one and the line stays there).
+template <int N>
+static constexpr int conv_threads(int lines)
+{
+    constexpr int T = FftPlanLow<N>::T;
+    return T <= 64 && (lines + 256 / T - 1) / (256 / T) < 256 ? 64 : 256;
+}
+
 int tild_conv_blocks(int nx, int ny, int nz)
 {
-    int T = 1;
-#define MFT_T(n_) if (nz == n_) T = FftPlanLow<n_>::T;
+    int B = 1;
+#define MFT_T(n_) if (nz == n_) B = conv_threads<n_>(nx * ny) / FftPlanLow<n_>::T;
     MFT_FOR_EACH_FFT_SIZE(MFT_T)
 #undef MFT_T
-    int B = 256 / T;
     return (nx * ny + B - 1) / B;
 }
 
@@ -287,41 +298,40 @@ constexpr bool conv_four_waves()
     return N == 32 || N == 64 || N == 128;
 }
 
-template <int N>
-static void launch_conv(TildEngine* e, float invM)
+template <int N, int NT>
+static void launch_conv_nt(TildEngine* e, float invM)
 {
     const mft_tild_desc& d = e->d;
-    constexpr int B = 256 / FftPlanLow<N>::T;
+    constexpr int B = NT / FftPlanLow<N>::T;
     const unsigned grid = (d.nx * d.ny + B - 1) / B;
     const float Mg = (float)((double)e->gvol * e->M);
     const float2* tw = fft_twiddles_device(N);
+    auto run = [&](auto* kernel) {
+        kernel<<<grid, NT, 0, e->stream>>>(e->S, e->Y, d.nx, d.ny, d.lx, d.ly, d.lz, e->kp, tw, invM, e->epart, Mg);
+    };
     bool done = false;
     if constexpr (conv_four_waves<N>()) {
-        if (e->nchan <= 2) {
-            k_conv_z<N, 2><<<grid, 256, 0, e->stream>>>(e->S, e->Y, d.nx, d.ny, d.lx, d.ly, d.lz, e->kp, tw, invM,
-                                                        e->epart, Mg);
-            done = true;
-        } else if (e->nchan == 3) {
-            k_conv_z<N, 3><<<grid, 256, 0, e->stream>>>(e->S, e->Y, d.nx, d.ny, d.lx, d.ly, d.lz, e->kp, tw, invM,
-                                                        e->epart, Mg);
-            done = true;
-        }
+        done = e->nchan <= 3;
+        if (e->nchan <= 2) run(k_conv_z<N, 2, NT>);
+        else if (e->nchan == 3) run(k_conv_z<N, 3, NT>);
     }
     if (done)
         ;
-    else if (e->nchan <= 2)
-        k_conv_z_wide<N, 2><<<grid, 256, 0, e->stream>>>(e->S, e->Y, d.nx, d.ny, d.lx, d.ly, d.lz, e->kp, tw, invM,
-                                                         e->epart, Mg);
-    else if (e->nchan == 3)
-        k_conv_z_wide<N, 3><<<grid, 256, 0, e->stream>>>(e->S, e->Y, d.nx, d.ny, d.lx, d.ly, d.lz, e->kp, tw, invM,
-                                                         e->epart, Mg);
-    else if (e->nchan <= 4)
-        k_conv_z_wide<N, 4><<<grid, 256, 0, e->stream>>>(e->S, e->Y, d.nx, d.ny, d.lx, d.ly, d.lz, e->kp, tw, invM,
-                                                         e->epart, Mg);
-    else
-        k_conv_z_wide<N, 8><<<grid, 256, 0, e->stream>>>(e->S, e->Y, d.nx, d.ny, d.lx, d.ly, d.lz, e->kp, tw, invM,
-                                                         e->epart, Mg);
+    else if (e->nchan <= 2) run(k_conv_z_wide<N, 2, NT>);
+    else if (e->nchan == 3) run(k_conv_z_wide<N, 3, NT>);
+    else if (e->nchan <= 4) run(k_conv_z_wide<N, 4, NT>);
+    else run(k_conv_z_wide<N, 8, NT>);
     if (e->kp.energy) k_energy_sum<<<d.npotentials, 256, 0, e->stream>>>(e->eout, e->epart, grid, d.npotentials);
+}
+
+template <int N>
+static void launch_conv(TildEngine* e, float invM)
+{
+    if (conv_threads<N>(e->d.nx * e->d.ny) == 64) {
+        if constexpr (FftPlanLow<N>::T <= 64) launch_conv_nt<N, 64>(e, invM);
+    } else {
+        launch_conv_nt<N, 256>(e, invM);
+    }
 }
 
 int tild_conv(TildEngine* e)

@@ -7,12 +7,11 @@ namespace mft {
 
 // Line transform of nfield grids along one axis.  Input real (float) or
 // complex, output complex or real part; scale applied on store.
-template <int N, int SIGN, bool REAL_IN, bool REAL_OUT>
+template <typename P, int SIGN, bool REAL_IN, bool REAL_OUT>
 __global__ void __launch_bounds__(256) k_fft_axis(const void* __restrict__ in, void* __restrict__ out, AxisGeom geom,
                                                   long field_stride, const float2* __restrict__ twg, float scale)
 {
-    using P = FftPlan<N>;
-    constexpr int T = P::T, E = P::E, B = 256 / T;
+    constexpr int N = P::N, T = P::T, E = P::E, B = 256 / T;
     __shared__ float2 lds[B * N];
     __shared__ float2 tw[N];
     for (int i = threadIdx.x; i < N; i += 256) tw[i] = twg[i];
@@ -37,7 +36,7 @@ __global__ void __launch_bounds__(256) k_fft_axis(const void* __restrict__ in, v
     }
     __syncthreads();
     LdsMap map{lline, B, inter, N};
-    line_fft<N, SIGN>(v, lds, tw, t, map);
+    line_fft_plan<P, SIGN>(v, lds, tw, t, map);
     if (!valid) return;
     if (REAL_OUT) {
         float* dst = (float*)out + field * field_stride + base;
@@ -60,7 +59,7 @@ __global__ void __launch_bounds__(256) k_fft_x_inv_packed(const float2* __restri
                                                           int ny, int nz, int nfield, int npk,
                                                           const float2* __restrict__ twg)
 {
-    using P = FftPlan<N>;
+    using P = FftPlanMesh<N>;
     constexpr int T = P::T, E = P::E, B = 256 / T;
     constexpr int NP = swz_pitch(N);
     __shared__ float2 lds[B * NP];
@@ -86,7 +85,7 @@ __global__ void __launch_bounds__(256) k_fft_x_inv_packed(const float2* __restri
     // a line's T threads are consecutive threads of one wavefront
     LdsMap map{lline, B, false, NP, true};
 #pragma unroll
-    for (int j = 0; j < 3; ++j) line_fft<N, +1, true>(pk[j], lds, tw, t, map);
+    for (int j = 0; j < 3; ++j) line_fft_plan<P, +1, true>(pk[j], lds, tw, t, map);
     if (!valid) return;
     // fields 2g (components in pk0.re, pk0.im, pk1.re) and 2g+1 (pk1.im,
     // pk2.re, pk2.im)
@@ -112,7 +111,7 @@ __global__ void __launch_bounds__(256) k_fft_x_fwd_tiles(const float* __restrict
                                                          float2* __restrict__ out, int ny, int nz, long cstride,
                                                          const float2* __restrict__ twg, int cover2)
 {
-    using P = FftPlan<N>;
+    using P = FftPlanMesh<N>;
     constexpr int T = P::T, E = P::E, B = 256 / T;
     constexpr int NP = swz_pitch(N);
     __shared__ float2 lds[B * NP];
@@ -274,7 +273,7 @@ __global__ void __launch_bounds__(256) k_fft_x_fwd_tiles(const float* __restrict
     for (int s = 0; s < E; ++s) v[s] = lds[lline * NP + t + T * s];
     // lines NP apart: each line's exchanges stay inside its own region
     LdsMap map{lline, B, false, NP, true};
-    line_fft<N, -1, true>(v, lds, tw, t, map);
+    line_fft_plan<P, -1, true>(v, lds, tw, t, map);
     if (line >= nlines) return;
     float2* dst = out + c * (long)N * nlines + (long)line * N;
 #pragma unroll
@@ -517,7 +516,7 @@ __global__ void __launch_bounds__(256) k_fft_x_fwd_tiles_staged(const float* __r
                                                                 long cstride, int ex0,
                                                                 const float2* __restrict__ twg)
 {
-    using P = FftPlan<N>;
+    using P = FftPlanMesh<N>;
     constexpr int T = P::T, E = P::E, B = 256 / T;
     extern __shared__ float4 stage4[];   // [2 z covers][B lines][2 y covers][ex0 / 4]
     float* stage = reinterpret_cast<float*>(stage4);
@@ -588,7 +587,7 @@ __global__ void __launch_bounds__(256) k_fft_x_fwd_tiles_staged(const float* __r
 #pragma unroll
     for (int s = 0; s < E; ++s) v[s] = lds[lline * N + t + T * s];
     LdsMap map{lline, B, false, N};
-    line_fft<N, -1, true>(v, lds, tw, t, map);
+    line_fft_plan<P, -1, true>(v, lds, tw, t, map);
     if (line >= nlines) return;
     float2* dst = out + c * (long)N * nlines + (long)line * N;
 #pragma unroll
@@ -600,7 +599,7 @@ __global__ void __launch_bounds__(256) k_fft_x_fwd_tiles_staged(const float* __r
 bool tild_x_fwd_staged_ok(int nx, int ex0, int maxcover)
 {
     int T = 0;
-#define MFT_T(n_) if (nx == n_) T = FftPlan<n_>::T;
+#define MFT_T(n_) if (nx == n_) T = FftPlanMesh<n_>::T;
     MFT_FOR_EACH_FFT_SIZE(MFT_T)
 #undef MFT_T
     if (T == 0 || ex0 % 4 != 0 || maxcover > 2) return false;
@@ -615,7 +614,7 @@ int tild_x_fwd_tiles(const float* tiles, const int* tab, float2* S, int nx, int 
         switch (nx) {
 #define MFT_CASE(n_)                                                                                      \
     case n_: {                                                                                            \
-        constexpr int B = 256 / FftPlan<n_>::T;                                                           \
+        constexpr int B = 256 / FftPlanMesh<n_>::T;                                                           \
         dim3 grid((ny * nz + B - 1) / B, nchan);                                                          \
         k_fft_x_fwd_tiles_staged<n_><<<grid, 256, 16 * B * (size_t)ex0, st>>>(tiles, tab, S, ny, nz, cstride, ex0, \
                                                                             fft_twiddles_device(n_));    \
@@ -631,7 +630,7 @@ int tild_x_fwd_tiles(const float* tiles, const int* tab, float2* S, int nx, int 
     switch (nx) {
 #define MFT_CASE(n_)                                                                                      \
     case n_: {                                                                                            \
-        constexpr int B = 256 / FftPlan<n_>::T;                                                           \
+        constexpr int B = 256 / FftPlanMesh<n_>::T;                                                           \
         dim3 grid((ny * nz + B - 1) / B, nchan);                                                          \
         k_fft_x_fwd_tiles<n_><<<grid, 256, 0, st>>>(tiles, tab, S, ny, nz, cstride, fft_twiddles_device(n_), \
                                                     cover2 ? 1 : 0);                                      \
@@ -645,20 +644,20 @@ int tild_x_fwd_tiles(const float* tiles, const int* tab, float2* S, int nx, int 
     return MFT_OK;
 }
 
-template <int N, int SIGN, bool RI, bool RO>
+template <typename P, int SIGN, bool RI, bool RO>
 static void launch_axis_n(const void* in, void* out, AxisGeom g, int nf, long fs, float scale, hipStream_t st)
 {
-    constexpr int B = 256 / FftPlan<N>::T;
+    constexpr int B = 256 / P::T;
     dim3 grid((g.nlines() + B - 1) / B, nf);
-    k_fft_axis<N, SIGN, RI, RO><<<grid, 256, 0, st>>>(in, out, g, fs, fft_twiddles_device(N), scale);
+    k_fft_axis<P, SIGN, RI, RO><<<grid, 256, 0, st>>>(in, out, g, fs, fft_twiddles_device(P::N), scale);
 }
 
-template <int SIGN, bool RI, bool RO>
+template <template <int> class Plan, int SIGN, bool RI, bool RO>
 static int launch_axis(const void* in, void* out, AxisGeom g, int nf, long fs, float scale, hipStream_t st)
 {
     switch (g.length()) {
 #define MFT_CASE(n_)                                                                                      \
-    case n_: launch_axis_n<n_, SIGN, RI, RO>(in, out, g, nf, fs, scale, st); break;
+    case n_: launch_axis_n<Plan<n_>, SIGN, RI, RO>(in, out, g, nf, fs, scale, st); break;
         MFT_FOR_EACH_FFT_SIZE(MFT_CASE)
 #undef MFT_CASE
     default:
@@ -669,16 +668,23 @@ static int launch_axis(const void* in, void* out, AxisGeom g, int nf, long fs, f
     return MFT_OK;
 }
 
-// the three variants the engine uses: forward real -> complex, forward and
-// inverse complex -> complex
+// the three variants in use: forward real -> complex, forward and inverse
+// complex -> complex
 int tild_axis(int sign, int real_in, int real_out, const void* in, void* out, AxisGeom g, int nf, long fs,
               float scale, hipStream_t st)
 {
-    if (sign < 0 && real_in && !real_out) return launch_axis<-1, true, false>(in, out, g, nf, fs, scale, st);
-    if (sign < 0 && !real_in && !real_out) return launch_axis<-1, false, false>(in, out, g, nf, fs, scale, st);
-    if (sign > 0 && !real_in && !real_out) return launch_axis<+1, false, false>(in, out, g, nf, fs, scale, st);
+    if (sign < 0 && real_in && !real_out) return launch_axis<FftPlan, -1, true, false>(in, out, g, nf, fs, scale, st);
+    if (sign < 0 && !real_in && !real_out) return launch_axis<FftPlan, -1, false, false>(in, out, g, nf, fs, scale, st);
+    if (sign > 0 && !real_in && !real_out) return launch_axis<FftPlan, +1, false, false>(in, out, g, nf, fs, scale, st);
     set_error(MFT_ERR_UNSUPPORTED, "axis pass variant not built");
     return MFT_ERR_UNSUPPORTED;
+}
+
+// the engine's y passes, complex to complex in place
+int tild_axis_mesh(int sign, float2* a, AxisGeom g, int nf, long fs, hipStream_t st)
+{
+    return sign < 0 ? launch_axis<FftPlanMesh, -1, false, false>(a, a, g, nf, fs, 1.0f, st)
+                    : launch_axis<FftPlanMesh, +1, false, false>(a, a, g, nf, fs, 1.0f, st);
 }
 
 int tild_x_inv_packed(const float2* Y, float4* F4, int nx, int ny, int nz, int nfield, hipStream_t st)
@@ -687,7 +693,7 @@ int tild_x_inv_packed(const float2* Y, float4* F4, int nx, int ny, int nz, int n
     switch (nx) {
 #define MFT_CASE(n_)                                                                                      \
     case n_: {                                                                                            \
-        constexpr int B = 256 / FftPlan<n_>::T;                                                           \
+        constexpr int B = 256 / FftPlanMesh<n_>::T;                                                           \
         dim3 grid((ny * nz + B - 1) / B, (nfield + 1) / 2);                                               \
         k_fft_x_inv_packed<n_><<<grid, 256, 0, st>>>(Y, F4, ny, nz, nfield, npk, fft_twiddles_device(n_)); \
         break;                                                                                            \
