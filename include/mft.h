@@ -323,13 +323,13 @@ int mft_tild_set_gather(mft_tild* eng, int variant);
  * in LDS; MFT_ERR_UNSUPPORTED where the grid does not allow the variant. */
 int mft_tild_set_grid_passes(mft_tild* eng, int variant);
 /* Replica groups (no counterpart in the reference, which steps one box):
- * independent TILD engines advanced together by one HIP graph holding eight
- * steps of every engine (each engine's kernels on its own stream, so the
- * replicas overlap on the device; remainders take ordinary steps).  Each engine gives the same bits as when
- * stepped alone.  Engines with potential ramps, DPD, Langevin potentials,
- * velocity Verlet or timing enabled, and a GJF engine's first step after its
- * state is set, take ordinary steps.  The engines stay owned by the caller;
- * destroy the group before them. */
+ * independent TILD engines advanced together.  Engines of one description (seed,
+ * bonds and state may differ) at the same step share every launch; the others
+ * step on their own streams.  Each engine gives the same bits as when stepped
+ * alone.  To share launches engines need GJF or EM, no grid line over 64 points,
+ * the default gather and grid passes, one charge per species, no ramps, bias,
+ * walls, angles, DPD or Langevin potentials, and timing off.  The engines stay
+ * owned by the caller; destroy the group before them. */
 typedef struct mft_tild_group mft_tild_group;
 int mft_tild_group_create(mft_tild_group** grp, mft_tild* const* engines, int n);
 int mft_tild_group_destroy(mft_tild_group* grp);

@@ -235,7 +235,6 @@ static int tild_setup(TildEngine* e)
     const int nconv_blocks = tild_conv_blocks(d.nx, d.ny, d.nz);
     if ((rc = dalloc(&e->epart, (size_t)nconv_blocks * kMaxPots))) return rc;
     if ((rc = dalloc(&e->eout, (size_t)kMaxPots + 1))) return rc;
-    if ((rc = dalloc(&e->d_step, (size_t)1))) return rc;
     if ((rc = dalloc(&e->bpart, (size_t)nblk(N)))) return rc;
     MFT_HIP(hipMemset(e->nBonds, 0, sizeof(int) * (size_t)N));
     MFT_HIP(hipMemset(e->bondedTo, 0, sizeof(int) * (size_t)N * mb));
@@ -522,7 +521,7 @@ static int do_steps(TildEngine* e, int nsteps, bool want_f, bool advance = true,
             // the next positions into their key order
             {
                 TimedScope ts(e, MFT_TK_SCAN);
-                if ((rc = tild_scan(e, true))) return rc;
+                if ((rc = tild_scan(e))) return rc;
             }
             TimedScope ts(e, MFT_TK_SCATTER);
             if ((rc = tild_permute(e))) return rc;
@@ -579,7 +578,7 @@ int mft_tild_destroy(mft_tild* e)
                     e->pio2, e->pio3, e->count, e->start, e->partial, e->rho, e->S, e->Y, e->F4, e->force_slot,
                     e->epart, e->eout, e->bpart, e->tiles, e->tile_tab, e->NA[0], e->NA[1], e->AT[0], e->AT[1],
                     e->AG[0], e->AG[1], e->nAngles, e->angleType, e->angleGroup, e->dcount, e->dstart,
-                    e->dcursor, e->dcell, e->dslots, e->fdpd, e->d_step};
+                    e->dcursor, e->dcell, e->dslots, e->fdpd};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (float* t : e->tables)
@@ -1127,115 +1126,129 @@ int mft_tild_num_outputs(mft_tild* e, int* nout)
 } // extern "C"
 
 // ------------------------------------------------- replica groups ---
-// Independent TILD systems advanced by one HIP graph: kGroupSteps steps of
-// every engine are captured once, each engine's launches on its own stream
-// between a fork from and a join back to the group's stream, so one graph
-// launch runs those steps of all replicas with their kernels overlapping on
-// the device.  The integrator reads the step index from device memory and the
-// key scan advances it, so a replay keys its noise by the steps it runs; an
-// even step count brings every engine's double buffers back to the captured
-// parity.  Engines
-// whose configuration a graph cannot replay (ramps, DPD, Langevin, velocity
-// Verlet, timing) and GJF engines whose previous noise is not yet keyed (the
-// first step after a state is set) take ordinary steps.
+// Independent TILD systems advanced together.  A small box's step is a dozen
+// launches of a few microseconds each, and the host submits one every 3 us
+// whatever stream or graph it goes to, so several such boxes cost as much as one
+// after the other.  Engines of one description (seeds and topologies may differ)
+// therefore share every launch: blockIdx.z picks the engine, its buffers come
+// from a table (8 replicas of 8.6 k particles on 24^3: 342 us a step of all from
+// a graph of their launches, 106 batched; 16 replicas 666 and 119).  Engines that differ from all
+// others, or whose step has more to it (a potential of its own kind of pass,
+// ramps, a grid line longer than the batched passes are built for), step on their
+// own streams.
 namespace mft {
 
-constexpr int kGroupSteps = 8;   // steps per graph replay (even)
-
-__global__ void k_set_step(uint32_t* __restrict__ d, uint32_t v) { *d = v; }
-
-static bool graph_ready(const TildEngine* e)
+// the engine's step consists of the batched passes alone
+static bool batch_ready(const TildEngine* e)
 {
     const mft_tild_desc& d = e->d;
     if (d.integrator != MFT_INT_GJF && d.integrator != MFT_INT_EM) return false;
-    if (e->dpd.on || e->lang.n || e->timing || e->nout == 0) return false;
+    if (std::max(d.nx, std::max(d.ny, d.nz)) > kBatchMaxGrid) return false;
+    if (e->dpd.on || e->lang.n || e->walls.n || !e->bias.empty() || d.maxangles > 0 || e->timing || e->nout == 0)
+        return false;
+    if (e->gather_mode != 1 || e->qslot >= 0 || e->plane_passes || e->xfwd_staged) return false;
     for (int p = 0; p < d.npotentials; ++p)
         if (e->pots[p].ramp) return false;
-    if (d.integrator == MFT_INT_GJF && !e->nz_keyed) return false;
     return true;
+}
+
+// the launches of a and b differ in buffers and seed only
+static bool same_step(const TildEngine* a, const TildEngine* b)
+{
+    const mft_tild_desc &p = a->d, &q = b->d;
+    if (p.nx != q.nx || p.ny != q.ny || p.nz != q.nz || p.lx != q.lx || p.ly != q.ly || p.lz != q.lz ||
+        p.pmeorder != q.pmeorder || p.nparticles != q.nparticles || p.nspecies != q.nspecies ||
+        p.maxbonds != q.maxbonds || p.npotentials != q.npotentials || p.integrator != q.integrator ||
+        p.delt != q.delt)
+        return false;
+    if (a->cur != b->cur || a->step != b->step || a->nz_keyed != b->nz_keyed || a->nchan != b->nchan ||
+        a->nforce != b->nforce || a->force_slot_h != b->force_slot_h || a->bp.ntypes != b->bp.ntypes ||
+        a->kp.fold != b->kp.fold)
+        return false;
+    for (int i = 0; i < p.npotentials; ++i) {
+        const mft_tild_potential &u = a->pots[i], &v = b->pots[i];
+        if (u.kind != v.kind || u.maskI != v.maskI || u.maskJ != v.maskJ || u.A != v.A || u.sigma != v.sigma ||
+            u.Rp != v.Rp)
+            return false;
+    }
+    for (int t = 0; t < a->bp.ntypes; ++t)
+        if (a->bp.k[t] != b->bp.k[t] || a->bp.r0[t] != b->bp.r0[t] || a->bp.style[t] != b->bp.style[t]) return false;
+    for (int s = 0; s < p.nspecies; ++s)
+        if (a->mass[s] != b->mass[s] || a->mob[s] != b->mob[s] || a->kp.qspec[s] != b->kp.qspec[s]) return false;
+    return true;
+}
+
+static StepPtrs step_ptrs(const TildEngine* e, int c)
+{
+    const int n = 1 - c;
+    return StepPtrs{e->X[c],  e->XO[c],  e->NZ[c],   e->X[n],  e->XO[n],   e->NZ[n],
+                    e->XN,    e->NN,     e->META[c], e->META[n], e->BS[c], e->BT[c],
+                    e->BS[n], e->BT[n],  e->key,     e->rank,  e->map,     e->start,
+                    e->partial, slot_count(e, c), slot_count(e, n), e->tiles, e->S, e->Y,
+                    e->F4,    e->fgrid,  e->d.seed};
+}
+
+// nsteps of the engines of one batch on the first one's stream
+static int batch_steps(const std::vector<TildEngine*>& eng, const TildBatch& b, int nsteps)
+{
+    TildEngine* e = eng[0];
+    const mft_tild_desc& d = e->d;
+    const AxisGeom gy{d.nx, d.ny, d.nz, 1};
+    const long cstride = (long)e->tg.ex[0] * e->tg.ex[1] * e->tg.ex[2];
+    int rc;
+    for (int i = 0; i < nsteps; ++i) {
+        const StepPtrs* tab = b.tab[e->cur];
+        if ((rc = tild_density(e, &b))) return rc;
+        if ((rc = tild_x_fwd_tiles(e->tiles, e->tile_tab, e->S, d.nx, d.ny, d.nz, e->nchan, cstride, e->stream,
+                                   e->tg.ex[0], false, e->tile_maxcover <= 2, tab, b.n)))
+            return rc;
+        if ((rc = tild_axis_mesh(-1, e->S, gy, e->nchan, e->M, e->stream, tab, b.n))) return rc;
+        if ((rc = tild_conv(e, &b))) return rc;
+        if ((rc = tild_axis_mesh(+1, e->Y, gy, e->npk, e->M, e->stream, tab, b.n))) return rc;
+        if ((rc = tild_x_inv_packed(e->Y, e->F4, d.nx, d.ny, d.nz, e->nout4, e->stream, tab, b.n))) return rc;
+        if ((rc = tild_gather(e, 1, &b))) return rc;
+        if ((rc = tild_integrate(e, false, &b))) return rc;
+        if ((rc = tild_scan(e, &b))) return rc;
+        if ((rc = tild_permute(e, &b))) return rc;
+        for (TildEngine* x : eng) {
+            x->cur = e->cur;
+            x->rho_valid = false;
+            if (d.integrator == MFT_INT_GJF) x->nz_keyed = true;
+            if (x->run_max > 0) x->run_pos++;
+            x->step++;
+        }
+    }
+    return MFT_OK;
 }
 
 } // namespace mft
 
 struct mft_tild_group {
     std::vector<mft_tild*> eng;
-    hipStream_t stream = nullptr;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    std::vector<int> cur0, gather0, plane0;   // what the graph was captured with
-    std::vector<int64_t> dstep_at;            // host step the device counter holds (-1: stale)
-    hipEvent_t fork = nullptr;
-    std::vector<hipEvent_t> join, pre, post;
+    StepPtrs* table = nullptr;       // [2][n] on the device
+    std::vector<StepPtrs> uploaded;  // what it holds
+    std::vector<hipEvent_t> ev;
 };
 
-static void group_drop_graph(mft_tild_group* g)
+// batches of the engines as they are now: indices into eng, first one leading
+static std::vector<std::vector<int>> group_batches(const mft_tild_group* g)
 {
-    if (g->exec) (void)hipGraphExecDestroy(g->exec);
-    if (g->graph) (void)hipGraphDestroy(g->graph);
-    g->exec = nullptr;
-    g->graph = nullptr;
-}
-
-// capture kGroupSteps steps of every engine into one graph (nothing runs;
-// the host bookkeeping the capture advanced is restored)
-static int group_capture(mft_tild_group* g)
-{
-    group_drop_graph(g);
-    const size_t n = g->eng.size();
-    std::vector<int64_t> step(n), run_pos(n);
-    std::vector<int> cur(n);
-    std::vector<bool> rho_valid(n), keyed(n);
-    for (size_t i = 0; i < n; ++i) {
-        TildEngine* e = g->eng[i];
-        step[i] = e->step;
-        run_pos[i] = e->run_pos;
-        cur[i] = e->cur;
-        rho_valid[i] = e->rho_valid;
-        keyed[i] = e->nz_keyed;
-        e->use_dstep = true;
+    std::vector<std::vector<int>> out;
+    for (int i = 0; i < (int)g->eng.size(); ++i) {
+        const TildEngine* e = g->eng[i];
+        bool joined = false;
+        if (batch_ready(e))
+            for (auto& b : out) {
+                const TildEngine* lead = g->eng[b[0]];
+                if (batch_ready(lead) && same_step(lead, e)) {
+                    b.push_back(i);
+                    joined = true;
+                    break;
+                }
+            }
+        if (!joined) out.push_back({i});
     }
-    int rc = MFT_OK;
-    hipError_t err = hipStreamBeginCapture(g->stream, hipStreamCaptureModeThreadLocal);
-    if (err == hipSuccess) err = hipEventRecord(g->fork, g->stream);
-    for (size_t i = 0; i < n && err == hipSuccess && rc == MFT_OK; ++i) {
-        TildEngine* e = g->eng[i];
-        err = hipStreamWaitEvent(e->stream, g->fork, 0);
-        if (err != hipSuccess) break;
-        rc = do_steps(e, kGroupSteps, false);
-        if (rc) break;
-        err = hipEventRecord(g->join[i], e->stream);
-        if (err == hipSuccess) err = hipStreamWaitEvent(g->stream, g->join[i], 0);
-    }
-    hipGraph_t graph = nullptr;
-    const hipError_t end = hipStreamEndCapture(g->stream, &graph);
-    for (size_t i = 0; i < n; ++i) {
-        TildEngine* e = g->eng[i];
-        e->use_dstep = false;
-        e->step = step[i];
-        e->run_pos = run_pos[i];
-        e->cur = cur[i];
-        e->rho_valid = rho_valid[i];
-        e->nz_keyed = keyed[i];
-    }
-    if (rc) {
-        if (graph) (void)hipGraphDestroy(graph);
-        return rc;
-    }
-    if (err == hipSuccess) err = end;
-    if (err == hipSuccess) err = hipGraphInstantiate(&g->exec, graph, nullptr, nullptr, 0);
-    if (err != hipSuccess) {
-        if (graph) (void)hipGraphDestroy(graph);
-        g->exec = nullptr;
-        set_error(MFT_ERR_DEVICE, "capturing the replica group's steps: %s", hipGetErrorString(err));
-        return MFT_ERR_DEVICE;
-    }
-    g->graph = graph;
-    for (size_t i = 0; i < n; ++i) {
-        g->cur0[i] = g->eng[i]->cur;
-        g->gather0[i] = g->eng[i]->gather_mode;
-        g->plane0[i] = g->eng[i]->plane_passes | (g->eng[i]->xfwd_staged << 1);
-    }
-    return MFT_OK;
+    return out;
 }
 
 extern "C" {
@@ -1250,24 +1263,15 @@ int mft_tild_group_create(mft_tild_group** out, mft_tild* const* engines, int n)
     }
     mft_tild_group* g = new mft_tild_group();
     g->eng.assign(engines, engines + n);
-    g->cur0.assign(n, -1);
-    g->gather0.assign(n, -1);
-    g->plane0.assign(n, -1);
-    g->dstep_at.assign(n, -1);
-    g->join.assign(n, nullptr);
-    g->pre.assign(n, nullptr);
-    g->post.assign(n, nullptr);
-    hipError_t err = hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking);
-    if (err == hipSuccess) err = hipEventCreateWithFlags(&g->fork, hipEventDisableTiming);
-    for (int i = 0; i < n && err == hipSuccess; ++i) {
-        err = hipEventCreateWithFlags(&g->join[i], hipEventDisableTiming);
-        if (err == hipSuccess) err = hipEventCreateWithFlags(&g->pre[i], hipEventDisableTiming);
-        if (err == hipSuccess) err = hipEventCreateWithFlags(&g->post[i], hipEventDisableTiming);
-    }
-    if (err != hipSuccess) {
+    g->ev.assign(n, nullptr);
+    int rc = dalloc(&g->table, 2 * (size_t)n);
+    hipError_t err = hipSuccess;
+    for (int i = 0; i < n && err == hipSuccess && !rc; ++i)
+        err = hipEventCreateWithFlags(&g->ev[i], hipEventDisableTiming);
+    if (rc || err != hipSuccess) {
         mft_tild_group_destroy(g);
-        set_error(MFT_ERR_DEVICE, "replica group set-up: %s", hipGetErrorString(err));
-        return MFT_ERR_DEVICE;
+        if (!rc) set_error(rc = MFT_ERR_DEVICE, "replica group set-up: %s", hipGetErrorString(err));
+        return rc;
     }
     *out = g;
     return MFT_OK;
@@ -1276,13 +1280,9 @@ int mft_tild_group_create(mft_tild_group** out, mft_tild* const* engines, int n)
 int mft_tild_group_destroy(mft_tild_group* g)
 {
     if (!g) return MFT_OK;
-    if (g->stream) (void)hipStreamSynchronize(g->stream);
-    group_drop_graph(g);
-    if (g->fork) (void)hipEventDestroy(g->fork);
-    for (auto* v : {&g->join, &g->pre, &g->post})
-        for (hipEvent_t ev : *v)
-            if (ev) (void)hipEventDestroy(ev);
-    if (g->stream) (void)hipStreamDestroy(g->stream);
+    for (hipEvent_t ev : g->ev)
+        if (ev) (void)hipEventDestroy(ev);
+    if (g->table) (void)hipFree(g->table);
     delete g;
     return MFT_OK;
 }
@@ -1292,66 +1292,48 @@ int mft_tild_group_step(mft_tild_group* g, int nsteps)
     MFT_REQUIRE(g && nsteps >= 0, MFT_ERR_INVALID, "bad argument");
     const size_t n = g->eng.size();
     for (size_t i = 0; i < n; ++i) MFT_REQUIRE(g->eng[i]->have_state, MFT_ERR_INVALID, "engine %zu has no state", i);
+    if (nsteps == 0) return MFT_OK;
     int rc;
-    int done = 0;
-    while (done < nsteps) {
-        bool ready = nsteps - done >= kGroupSteps;
-        for (size_t i = 0; i < n && ready; ++i) ready = graph_ready(g->eng[i]);
-        if (!ready) {
-            // one ordinary step of every engine, each on its own stream
-            for (size_t i = 0; i < n; ++i) {
-                if ((rc = do_steps(g->eng[i], 1, false))) return rc;
-                g->dstep_at[i] = -1;
-            }
-            ++done;
-            continue;
-        }
-        bool same = g->exec != nullptr;
-        for (size_t i = 0; i < n && same; ++i) {
-            const TildEngine* e = g->eng[i];
-            same = g->gather0[i] == e->gather_mode && g->plane0[i] == (e->plane_passes | (e->xfwd_staged << 1));
-        }
-        if (!same && (rc = group_capture(g))) return rc;
-        bool parity = true;
-        for (size_t i = 0; i < n; ++i) parity = parity && g->eng[i]->cur == g->cur0[i];
-        if (!parity) {
-            // an odd number of ordinary steps since the capture: one more
-            for (size_t i = 0; i < n; ++i) {
-                if ((rc = do_steps(g->eng[i], 1, false))) return rc;
-                g->dstep_at[i] = -1;
-            }
-            ++done;
-            continue;
-        }
-        // each engine's earlier work and device step index before the replay
-        for (size_t i = 0; i < n; ++i) {
-            TildEngine* e = g->eng[i];
-            if (g->dstep_at[i] != e->step) {
-                k_set_step<<<1, 1, 0, e->stream>>>(e->d_step, (uint32_t)e->step);
-                MFT_LAUNCH_CHECK();
-            }
-            MFT_HIP(hipEventRecord(g->pre[i], e->stream));
-            MFT_HIP(hipStreamWaitEvent(g->stream, g->pre[i], 0));
-        }
-        MFT_HIP(hipGraphLaunch(g->exec, g->stream));
-        for (size_t i = 0; i < n; ++i) {
-            TildEngine* e = g->eng[i];
-            MFT_HIP(hipEventRecord(g->post[i], g->stream));
-            MFT_HIP(hipStreamWaitEvent(e->stream, g->post[i], 0));
-            e->step += kGroupSteps;
-            if (e->run_max > 0) e->run_pos += kGroupSteps;
-            e->rho_valid = false;
-            g->dstep_at[i] = e->step;
-        }
-        done += kGroupSteps;
+    const std::vector<std::vector<int>> batches = group_batches(g);
+    // the batches' buffer tables, uploaded again when an engine's buffers or the
+    // batches changed (set_topology allocates anew)
+    std::vector<StepPtrs> want;
+    for (int c = 0; c < 2; ++c)
+        for (const auto& b : batches)
+            for (int i : b) want.push_back(step_ptrs(g->eng[i], c));
+    if (g->uploaded.size() != want.size() ||
+        std::memcmp(g->uploaded.data(), want.data(), sizeof(StepPtrs) * want.size()) != 0) {
+        for (mft_tild* e : g->eng) MFT_HIP(hipStreamSynchronize(e->stream));
+        MFT_HIP(hipMemcpy(g->table, want.data(), sizeof(StepPtrs) * want.size(), hipMemcpyHostToDevice));
+        g->uploaded = want;
     }
+    // a lead's stream runs after the work its members already have on theirs
+    size_t first = 0;
+    for (const auto& b : batches) {
+        if (b.size() > 1) {
+            std::vector<TildEngine*> eng;
+            for (int i : b) eng.push_back(g->eng[i]);
+            for (size_t k = 1; k < b.size(); ++k) {
+                MFT_HIP(hipEventRecord(g->ev[b[k]], eng[k]->stream));
+                MFT_HIP(hipStreamWaitEvent(eng[0]->stream, g->ev[b[k]], 0));
+            }
+            const TildBatch tb{{g->table + first, g->table + n + first}, (int)b.size()};
+            if ((rc = batch_steps(eng, tb, nsteps))) return rc;
+            MFT_HIP(hipEventRecord(g->ev[b[0]], eng[0]->stream));
+            for (size_t k = 1; k < b.size(); ++k) MFT_HIP(hipStreamWaitEvent(eng[k]->stream, g->ev[b[0]], 0));
+        }
+        first += b.size();
+    }
+    // the others' steps one after the other: their streams overlap on the device
+    for (int s = 0; s < nsteps; ++s)
+        for (const auto& b : batches)
+            if (b.size() == 1 && (rc = do_steps(g->eng[b[0]], 1, false))) return rc;
     return MFT_OK;
 }
 
 int mft_tild_group_synchronize(mft_tild_group* g)
 {
     MFT_REQUIRE(g, MFT_ERR_INVALID, "null argument");
-    MFT_HIP(hipStreamSynchronize(g->stream));
     for (mft_tild* e : g->eng) MFT_HIP(hipStreamSynchronize(e->stream));
     return MFT_OK;
 }

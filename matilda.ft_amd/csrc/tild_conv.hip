@@ -240,20 +240,28 @@ __device__ __forceinline__ void conv_z_body(const float2* __restrict__ S, float2
 
 // Up to three channels the pass fits 128 registers (four waves per SIMD);
 // more channels keep the register count they need.
-template <int N, int NCH, int NT>
+template <int N, int NCH, int NT, bool BATCH = false>
 __global__ void __launch_bounds__(NT, 4) k_conv_z(const float2* __restrict__ S, float2* __restrict__ Y, int nx, int ny,
                                                 float Lx, float Ly, float Lz, KParams kp, const float2* __restrict__ twg,
-                                                float invM, double* __restrict__ epart, float Mgvol)
+                                                float invM, double* __restrict__ epart, float Mgvol, const StepPtrs* __restrict__ tab)
 {
+    if constexpr (BATCH) {
+        S = batch_global(batch_ptrs(tab)->S);
+        Y = batch_global(batch_ptrs(tab)->Y);
+    }
     conv_z_body<N, NCH, NT>(S, Y, nx, ny, Lx, Ly, Lz, kp, twg, invM, epart, Mgvol);
 }
 
-template <int N, int NCH, int NT>
+template <int N, int NCH, int NT, bool BATCH = false>
 __global__ void __launch_bounds__(NT) k_conv_z_wide(const float2* __restrict__ S, float2* __restrict__ Y, int nx,
                                                      int ny, float Lx, float Ly, float Lz, KParams kp,
                                                      const float2* __restrict__ twg, float invM,
-                                                     double* __restrict__ epart, float Mgvol)
+                                                     double* __restrict__ epart, float Mgvol, const StepPtrs* __restrict__ tab)
 {
+    if constexpr (BATCH) {
+        S = batch_global(batch_ptrs(tab)->S);
+        Y = batch_global(batch_ptrs(tab)->Y);
+    }
     conv_z_body<N, NCH, NT>(S, Y, nx, ny, Lx, Ly, Lz, kp, twg, invM, epart, Mgvol);
 }
 
@@ -299,7 +307,7 @@ constexpr bool conv_four_waves()
 }
 
 template <int N, int NT>
-static void launch_conv_nt(TildEngine* e, float invM)
+static void launch_conv_nt(TildEngine* e, float invM, const TildBatch* b)
 {
     const mft_tild_desc& d = e->d;
     constexpr int B = NT / FftPlanLow<N>::T;
@@ -307,8 +315,22 @@ static void launch_conv_nt(TildEngine* e, float invM)
     const float Mg = (float)((double)e->gvol * e->M);
     const float2* tw = fft_twiddles_device(N);
     auto run = [&](auto* kernel) {
-        kernel<<<grid, NT, 0, e->stream>>>(e->S, e->Y, d.nx, d.ny, d.lx, d.ly, d.lz, e->kp, tw, invM, e->epart, Mg);
+        kernel<<<dim3(grid, 1, b ? b->n : 1), NT, 0, e->stream>>>(e->S, e->Y, d.nx, d.ny, d.lx, d.ly, d.lz, e->kp, tw,
+                                                                  invM, e->epart, Mg, b ? b->tab[e->cur] : nullptr);
     };
+    constexpr bool many = N <= kBatchMaxGrid;
+    if (b) {
+        if constexpr (many && conv_four_waves<N>()) {
+            if (e->nchan <= 2) return run(k_conv_z<N, 2, NT, many>);
+            if (e->nchan == 3) return run(k_conv_z<N, 3, NT, many>);
+        }
+        if constexpr (many) {
+            if (e->nchan <= 2) return run(k_conv_z_wide<N, 2, NT, many>);
+            if (e->nchan == 3) return run(k_conv_z_wide<N, 3, NT, many>);
+            if (e->nchan <= 4) return run(k_conv_z_wide<N, 4, NT, many>);
+            return run(k_conv_z_wide<N, 8, NT, many>);
+        }
+    }
     bool done = false;
     if constexpr (conv_four_waves<N>()) {
         done = e->nchan <= 3;
@@ -325,22 +347,22 @@ static void launch_conv_nt(TildEngine* e, float invM)
 }
 
 template <int N>
-static void launch_conv(TildEngine* e, float invM)
+static void launch_conv(TildEngine* e, float invM, const TildBatch* b)
 {
     if (conv_threads<N>(e->d.nx * e->d.ny) == 64) {
-        if constexpr (FftPlanLow<N>::T <= 64) launch_conv_nt<N, 64>(e, invM);
+        if constexpr (FftPlanLow<N>::T <= 64) launch_conv_nt<N, 64>(e, invM, b);
     } else {
-        launch_conv_nt<N, 256>(e, invM);
+        launch_conv_nt<N, 256>(e, invM, b);
     }
 }
 
-int tild_conv(TildEngine* e)
+int tild_conv(TildEngine* e, const TildBatch* b)
 {
     const mft_tild_desc& d = e->d;
     float invM = 1.0f / (float)e->M;
     switch (d.nz) {
 #define MFT_CASE(n_)                                                                                      \
-    case n_: launch_conv<n_>(e, invM); break;
+    case n_: launch_conv<n_>(e, invM, b); break;
         MFT_FOR_EACH_FFT_SIZE(MFT_CASE)
 #undef MFT_CASE
     default: return MFT_ERR_UNSUPPORTED;

@@ -7,10 +7,13 @@ namespace mft {
 
 // Line transform of nfield grids along one axis.  Input real (float) or
 // complex, output complex or real part; scale applied on store.
-template <typename P, int SIGN, bool REAL_IN, bool REAL_OUT>
+template <typename P, int SIGN, bool REAL_IN, bool REAL_OUT, bool BATCH = false>
 __global__ void __launch_bounds__(256) k_fft_axis(const void* __restrict__ in, void* __restrict__ out, AxisGeom geom,
-                                                  long field_stride, const float2* __restrict__ twg, float scale)
+                                                  long field_stride, const float2* __restrict__ twg, float scale,
+                                                  const StepPtrs* __restrict__ tab = nullptr)
 {
+    if constexpr (BATCH) // in place: the spectra forward, the packed forces back
+        in = out = batch_global(SIGN < 0 ? batch_ptrs(tab)->S : batch_ptrs(tab)->Y);
     constexpr int N = P::N, T = P::T, E = P::E, B = 256 / T;
     __shared__ float2 lds[B * N];
     __shared__ float2 tw[N];
@@ -54,11 +57,16 @@ __global__ void __launch_bounds__(256) k_fft_axis(const void* __restrict__ in, v
 // field r/2 for even r, the imaginary part for odd r); one workgroup row
 // transforms the three packed lines of fields 2g and 2g+1 and writes them as
 // float4 (x, y, z, 0).
-template <int N>
+template <int N, bool BATCH = false>
 __global__ void __launch_bounds__(256) k_fft_x_inv_packed(const float2* __restrict__ Y, float4* __restrict__ F4,
                                                           int ny, int nz, int nfield, int npk,
-                                                          const float2* __restrict__ twg)
+                                                          const float2* __restrict__ twg,
+                                                          const StepPtrs* __restrict__ tab)
 {
+    if constexpr (BATCH) {
+        Y = batch_global(batch_ptrs(tab)->Y);
+        F4 = batch_global(batch_ptrs(tab)->F4);
+    }
     using P = FftPlanMesh<N>;
     constexpr int T = P::T, E = P::E, B = 256 / T;
     constexpr int NP = swz_pitch(N);
@@ -106,11 +114,16 @@ __global__ void __launch_bounds__(256) k_fft_x_inv_packed(const float2* __restri
 // and the offsets of the covering tile entries.  The block's B lines are
 // summed into LDS first (consecutive lanes on consecutive x, so the tile rows
 // are read coalesced), then transformed from there.
-template <int N>
+template <int N, bool BATCH = false>
 __global__ void __launch_bounds__(256) k_fft_x_fwd_tiles(const float* __restrict__ tiles, const int* __restrict__ tab,
                                                          float2* __restrict__ out, int ny, int nz, long cstride,
-                                                         const float2* __restrict__ twg, int cover2)
+                                                         const float2* __restrict__ twg, int cover2,
+                                                         const StepPtrs* __restrict__ btab)
 {
+    if constexpr (BATCH) {
+        tiles = batch_global(batch_ptrs(btab)->tiles);
+        out = batch_global(batch_ptrs(btab)->S);
+    }
     using P = FftPlanMesh<N>;
     constexpr int T = P::T, E = P::E, B = 256 / T;
     constexpr int NP = swz_pitch(N);
@@ -608,7 +621,7 @@ bool tild_x_fwd_staged_ok(int nx, int ex0, int maxcover)
 }
 
 int tild_x_fwd_tiles(const float* tiles, const int* tab, float2* S, int nx, int ny, int nz, int nchan, long cstride,
-                     hipStream_t st, int ex0, bool staged, bool cover2)
+                     hipStream_t st, int ex0, bool staged, bool cover2, const StepPtrs* btab, int nbatch)
 {
     if (staged) {
         switch (nx) {
@@ -631,9 +644,10 @@ int tild_x_fwd_tiles(const float* tiles, const int* tab, float2* S, int nx, int 
 #define MFT_CASE(n_)                                                                                      \
     case n_: {                                                                                            \
         constexpr int B = 256 / FftPlanMesh<n_>::T;                                                           \
-        dim3 grid((ny * nz + B - 1) / B, nchan);                                                          \
-        k_fft_x_fwd_tiles<n_><<<grid, 256, 0, st>>>(tiles, tab, S, ny, nz, cstride, fft_twiddles_device(n_), \
-                                                    cover2 ? 1 : 0);                                      \
+        dim3 grid((ny * nz + B - 1) / B, nchan, nbatch);                                                  \
+        constexpr bool many = n_ <= kBatchMaxGrid;                                                        \
+        (btab && many ? k_fft_x_fwd_tiles<n_, many> : k_fft_x_fwd_tiles<n_>)<<<grid, 256, 0, st>>>(       \
+            tiles, tab, S, ny, nz, cstride, fft_twiddles_device(n_), cover2 ? 1 : 0, btab);               \
         break;                                                                                            \
     }
         MFT_FOR_EACH_FFT_SIZE(MFT_CASE)
@@ -680,22 +694,51 @@ int tild_axis(int sign, int real_in, int real_out, const void* in, void* out, Ax
     return MFT_ERR_UNSUPPORTED;
 }
 
-// the engine's y passes, complex to complex in place
-int tild_axis_mesh(int sign, float2* a, AxisGeom g, int nf, long fs, hipStream_t st)
+template <int N, int SIGN>
+static void launch_axis_batch(AxisGeom g, int nf, long fs, hipStream_t st, const StepPtrs* tab, int nbatch)
 {
+    if constexpr (N <= kBatchMaxGrid) {
+        using P = FftPlanMesh<N>;
+        constexpr int B = 256 / P::T;
+        dim3 grid((g.nlines() + B - 1) / B, nf, nbatch);
+        k_fft_axis<P, SIGN, false, false, true><<<grid, 256, 0, st>>>(nullptr, nullptr, g, fs, fft_twiddles_device(N),
+                                                                      1.0f, tab);
+    }
+}
+
+// the engine's y passes, complex to complex in place
+int tild_axis_mesh(int sign, float2* a, AxisGeom g, int nf, long fs, hipStream_t st, const StepPtrs* tab, int nbatch)
+{
+    if (tab) {
+        switch (g.length()) {
+#define MFT_CASE(n_)                                                                                      \
+    case n_:                                                                                              \
+        if (sign < 0) launch_axis_batch<n_, -1>(g, nf, fs, st, tab, nbatch);                              \
+        else launch_axis_batch<n_, +1>(g, nf, fs, st, tab, nbatch);                                       \
+        break;
+            MFT_FOR_EACH_FFT_SIZE(MFT_CASE)
+#undef MFT_CASE
+        default: return MFT_ERR_UNSUPPORTED;
+        }
+        MFT_LAUNCH_CHECK();
+        return MFT_OK;
+    }
     return sign < 0 ? launch_axis<FftPlanMesh, -1, false, false>(a, a, g, nf, fs, 1.0f, st)
                     : launch_axis<FftPlanMesh, +1, false, false>(a, a, g, nf, fs, 1.0f, st);
 }
 
-int tild_x_inv_packed(const float2* Y, float4* F4, int nx, int ny, int nz, int nfield, hipStream_t st)
+int tild_x_inv_packed(const float2* Y, float4* F4, int nx, int ny, int nz, int nfield, hipStream_t st,
+                      const StepPtrs* tab, int nbatch)
 {
     const int npk = (3 * nfield + 1) / 2;
     switch (nx) {
 #define MFT_CASE(n_)                                                                                      \
     case n_: {                                                                                            \
         constexpr int B = 256 / FftPlanMesh<n_>::T;                                                           \
-        dim3 grid((ny * nz + B - 1) / B, (nfield + 1) / 2);                                               \
-        k_fft_x_inv_packed<n_><<<grid, 256, 0, st>>>(Y, F4, ny, nz, nfield, npk, fft_twiddles_device(n_)); \
+        dim3 grid((ny * nz + B - 1) / B, (nfield + 1) / 2, nbatch);                                       \
+        constexpr bool many = n_ <= kBatchMaxGrid;                                                        \
+        (tab && many ? k_fft_x_inv_packed<n_, many> : k_fft_x_inv_packed<n_>)<<<grid, 256, 0, st>>>(      \
+            Y, F4, ny, nz, nfield, npk, fft_twiddles_device(n_), tab);                                    \
         break;                                                                                            \
     }
         MFT_FOR_EACH_FFT_SIZE(MFT_CASE)

@@ -252,11 +252,6 @@ struct TildEngine {
     // a GJF step of this engine; the integrator then regenerates it instead of
     // reading NZ, and NZ is not carried through the permutation
     bool nz_keyed = false;
-    // step index on the device for graph-captured steps: the integrator
-    // reads it and the key scan advances it, so replays key their noise by
-    // the step they run (null kernel argument on the ordinary path)
-    uint32_t* d_step = nullptr;
-    bool use_dstep = false;
     // step temporaries in slot order
     float4 *XN = nullptr, *NN = nullptr; // next positions (12 bytes a slot: ff_load / ff_store) and noise
     float4* fgrid = nullptr;             // grid force per slot, 12 bytes a slot (ff_load / ff_store)
@@ -335,6 +330,39 @@ struct TildEngine {
 // types are neither carried through the permutation nor read.
 inline int* slot_bond_types(const TildEngine* e, int c) { return e->bp.ntypes > 1 ? e->BT[c] : nullptr; }
 
+// The buffers a step from buffer c reads and writes, for kernels that advance
+// several engines of one description by one launch: blockIdx.z picks the engine.
+struct StepPtrs {
+    float4 *X, *XO, *NZ, *X2, *XO2, *NZ2, *XN, *NN;
+    PMeta *META, *META2;
+    int *BS, *BT, *BS2, *BT2;
+    int *key, *rank, *map, *start, *partial, *count, *other;
+    float* tiles;
+    float2 *S, *Y;
+    float4 *F4, *fgrid;
+    uint64_t seed;
+};
+// n engines (tab[c]: their buffers when they step from buffer c) on one stream;
+// every launcher below takes the first of them and, for more than one, this.
+struct TildBatch {
+    const StepPtrs* tab[2];
+    int n;
+};
+
+// Entries of the table are scalar loads, and its pointers are global memory (which
+// the compiler cannot see: the accesses would be flat).
+template <typename T>
+__device__ __forceinline__ T* batch_global(T* p)
+{
+    return (T*)(__attribute__((address_space(1))) T*)p;
+}
+typedef const __attribute__((address_space(4))) StepPtrs* StepPtrsRef;
+__device__ __forceinline__ StepPtrsRef batch_ptrs(const StepPtrs* tab) { return (StepPtrsRef)tab + blockIdx.z; }
+
+// Longest line the batched passes are built for: a batch is there for boxes that
+// are too small to fill the chip by themselves.
+constexpr int kBatchMaxGrid = 64;
+
 // key counts of the step that starts from buffer c
 inline int* slot_count(const TildEngine* e, int c) { return e->count + (size_t)c * e->nkeys; }
 
@@ -360,29 +388,32 @@ static int dalloc(T** p, size_t n)
 // ---- grid passes (tild_grid.hip, tild_conv.hip) ----
 int tild_axis(int sign, int real_in, int real_out, const void* in, void* out, AxisGeom g, int nf, long fs,
               float scale, hipStream_t st);
-int tild_axis_mesh(int sign, float2* a, AxisGeom g, int nf, long fs, hipStream_t st);
+int tild_axis_mesh(int sign, float2* a, AxisGeom g, int nf, long fs, hipStream_t st,
+                   const StepPtrs* tab = nullptr, int nbatch = 1);
 int tild_x_fwd_tiles(const float* tiles, const int* tab, float2* S, int nx, int ny, int nz, int nchan, long cstride,
-                     hipStream_t st, int ex0 = 0, bool staged = false, bool cover2 = false);
+                     hipStream_t st, int ex0 = 0, bool staged = false, bool cover2 = false,
+                     const StepPtrs* btab = nullptr, int nbatch = 1);
 bool tild_x_fwd_staged_ok(int nx, int ex0, int maxcover);
-int tild_x_inv_packed(const float2* Y, float4* F4, int nx, int ny, int nz, int nfield, hipStream_t st);
+int tild_x_inv_packed(const float2* Y, float4* F4, int nx, int ny, int nz, int nfield, hipStream_t st,
+                      const StepPtrs* tab = nullptr, int nbatch = 1);
 bool tild_plane_supported(int nx, int ny);
 int tild_xy_fwd_tiles_plane(const float* tiles, const int* tab, float2* S, int nx, int ny, int nz, int nchan,
                             long cstride, hipStream_t st);
 int tild_yx_inv_packed_plane(const float2* Y, float4* F4, int nx, int ny, int nz, int nfield, hipStream_t st);
 int tild_conv_blocks(int nx, int ny, int nz);
-int tild_conv(TildEngine* e);
+int tild_conv(TildEngine* e, const TildBatch* b = nullptr);
 
 // ---- particle passes (tild_particles.hip) ----
 int tild_tiles_configure(TildEngine* e); // brick geometry, LDS sizes, tile tables
 int tild_sort_state(TildEngine* e);     // particle-id-order staging -> key order
 int tild_unsort(TildEngine* e, int what); // key order -> particle-id-order staging
-int tild_scan(TildEngine* e, bool advance_step = false);
-int tild_permute(TildEngine* e);         // next positions into the next key order
-int tild_density(TildEngine* e);          // tiles of the current positions
+int tild_scan(TildEngine* e, const TildBatch* b = nullptr);
+int tild_permute(TildEngine* e, const TildBatch* b = nullptr); // next positions into the next key order
+int tild_density(TildEngine* e, const TildBatch* b = nullptr); // tiles of the current positions
 int tild_density_reduce(TildEngine* e);   // tiles -> rho (when the densities are read)
-int tild_gather(TildEngine* e, int mode);
+int tild_gather(TildEngine* e, int mode, const TildBatch* b = nullptr);
 bool tild_gather_brick_fits(const TildEngine* e);   // gather variant 2's windows fit in LDS
-int tild_integrate(TildEngine* e, bool want_f);
+int tild_integrate(TildEngine* e, bool want_f, const TildBatch* b = nullptr);
 void erf_table(int kind, double sigma, double Rp, int nx, int ny, int nz, float lx, float ly, float lz,
                std::vector<float>& out);
 int tild_bond_energy(TildEngine* e);

@@ -316,8 +316,14 @@ __global__ void k_unsort(float* __restrict__ out, const float4* __restrict__ src
     out[id * 3 + 2] = v.z;
 }
 
-__global__ void k_scan_reduce(const int* __restrict__ count, int M, int* __restrict__ partial)
+template <bool BATCH>
+__global__ void k_scan_reduce(const int* __restrict__ count, int M, int* __restrict__ partial,
+                              const StepPtrs* __restrict__ tab)
 {
+    if constexpr (BATCH) {
+        count = batch_global(batch_ptrs(tab)->count);
+        partial = batch_global(batch_ptrs(tab)->partial);
+    }
     __shared__ int sh[16];
     long base = (long)blockIdx.x * kScanChunk;
     int s = 0;
@@ -339,10 +345,18 @@ static_assert(kScanItems == 16, "four int4 per thread");
 // alternate between steps: `other`, read by the previous step's scan, is cleared
 // here for the next one.  Each block adds the totals of the blocks before it (at
 // most a few thousand values, read from L2); one block needs none.
+template <bool BATCH>
 __global__ void k_scan_apply(const int* __restrict__ count, int* __restrict__ other, int M,
                              const int* __restrict__ partial, int* __restrict__ start, int ns,
-                             uint32_t* __restrict__ dstep)
+                             const StepPtrs* __restrict__ tab)
 {
+    if constexpr (BATCH) {
+        const auto B = batch_ptrs(tab);
+        count = batch_global(B->count);
+        other = batch_global(B->other);
+        partial = batch_global(B->partial);
+        start = batch_global(B->start);
+    }
     __shared__ int sh[16];
     const long first = (long)blockIdx.x * blockDim.x * kScanItems;
     int c = 0;
@@ -373,24 +387,38 @@ __global__ void k_scan_apply(const int* __restrict__ count, int* __restrict__ ot
             reinterpret_cast<int4*>(other + base)[k] = make_int4(0, 0, 0, 0);
         }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        start[M] = ns;
-        // the step's last reader of the device step index ran before this
-        // scan (the integrator): advance it for the next step
-        if (dstep) *dstep += 1u;
-    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) start[M] = ns;
 }
 
 // Particle state into the next step's key order: the slot's next position
 // and noise (from the integrator), its current position as the next previous
 // position, identity and bonds; map[slot] = new slot.  BT/BT2 null: a single
 // bond type, whose slots' types are not carried (every bond is type 0).
+template <bool BATCH>
 __global__ void k_permute(int ns, int maxbonds, const int* __restrict__ key, const int* __restrict__ rank,
                           const int* __restrict__ start, int* __restrict__ map, const float4* __restrict__ XN,
                           const float4* __restrict__ NN, const float4* __restrict__ X, const PMeta* __restrict__ META,
                           const int* __restrict__ BT, float4* __restrict__ X2, float4* __restrict__ XO2,
-                          float4* __restrict__ NZ2, PMeta* __restrict__ META2, int* __restrict__ BT2)
+                          float4* __restrict__ NZ2, PMeta* __restrict__ META2, int* __restrict__ BT2,
+                          const StepPtrs* __restrict__ tab)
 {
+    if constexpr (BATCH) {
+        const auto B = batch_ptrs(tab);
+        key = batch_global(B->key);
+        rank = batch_global(B->rank);
+        start = batch_global(B->start);
+        map = batch_global(B->map);
+        XN = batch_global(B->XN);
+        if (NN) NN = batch_global(B->NN);
+        X = batch_global(B->X);
+        META = batch_global(B->META);
+        if (BT2) BT = batch_global(B->BT);
+        X2 = batch_global(B->X2);
+        XO2 = batch_global(B->XO2);
+        NZ2 = batch_global(B->NZ2);
+        META2 = batch_global(B->META2);
+        if (BT2) BT2 = batch_global(B->BT2);
+    }
     int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= ns) return;
     const int n = start[key[s]] + rank[s];
@@ -406,9 +434,16 @@ __global__ void k_permute(int ns, int maxbonds, const int* __restrict__ key, con
 }
 
 // bond partner slots into the new order (after every map entry is written)
+template <bool BATCH>
 __global__ void k_remap_bonds(int ns, int maxbonds, const int* __restrict__ map, const int* __restrict__ BS,
-                              int* __restrict__ BS2)
+                              int* __restrict__ BS2, const StepPtrs* __restrict__ tab)
 {
+    if constexpr (BATCH) {
+        const auto B = batch_ptrs(tab);
+        map = batch_global(B->map);
+        BS = batch_global(B->BS);
+        BS2 = batch_global(B->BS2);
+    }
     int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= ns) return;
     const int n = map[s];
@@ -602,12 +637,18 @@ struct TileWalk {
 // One workgroup per brick: the brick's particles (contiguous in key order)
 // spread their (p+1)^3 weights over the brick's tile in LDS in fixed point;
 // the tile is written as float times 1/gvol.
-template <int P, int BM>
+template <int P, int BM, bool BATCH>
 __global__ void __launch_bounds__(kTileThreads) k_density_tile(
     float* __restrict__ tiles, int nchan, int qchan, const float4* __restrict__ spos,
     const int* __restrict__ start, TileGeom tg, int nx, int ny, int nz, float dx0, float dx1, float dx2,
-    double inv_gvol)
+    double inv_gvol, const StepPtrs* __restrict__ tab)
 {
+    if constexpr (BATCH) {
+        const auto B = batch_ptrs(tab);
+        tiles = batch_global(B->tiles);
+        spos = batch_global(B->X);
+        start = batch_global(B->start);
+    }
     constexpr int TP = BM + P, T3 = TP * TP * TP;
     extern __shared__ unsigned long long acc64[]; // [nchan][T3] (32-bit words in the narrow case)
     unsigned int* acc32 = reinterpret_cast<unsigned int*>(acc64);
@@ -860,12 +901,19 @@ struct GatherMap {
 // contiguous in key order; the workgroup stages that species' force field
 // window and writes the particles' grid forces (zero for a species no
 // potential acts on).
-template <int P, int BM>
+template <int P, int BM, bool BATCH>
 __global__ void __launch_bounds__(kTileThreads) k_gather_species(
     float4* __restrict__ fgrid, const float4* __restrict__ F4, GatherMap gm, const float4* __restrict__ spos,
     const PMeta* __restrict__ smeta, const int* __restrict__ start, TileGeom tg, int nx, int ny, int nz, float dx0,
-    float dx1, float dx2)
+    float dx1, float dx2, const StepPtrs* __restrict__ tab)
 {
+    if constexpr (BATCH) {
+        const auto B = batch_ptrs(tab);
+        fgrid = batch_global(B->fgrid);
+        F4 = batch_global(B->F4);
+        spos = batch_global(B->X);
+        start = batch_global(B->start);
+    }
     constexpr int TP = BM + P, T3 = TP * TP * TP;
     __shared__ Win3 ft[T3];
     __shared__ int xg[TP], yo[TP], zo[TP];
@@ -1333,10 +1381,10 @@ __device__ __forceinline__ SpeciesCoef species_coef(const StepArgs& A, int ty)
 
 __device__ __forceinline__ int integrate_slot(int s, float4 xc, PMeta meta, const float* fo, const StepArgs& A,
                                               uint32_t step, const TileGeom& tg, float4 xo4, float4 nz4,
-                                              const SpeciesCoef& sc)
+                                              const SpeciesCoef& sc, uint64_t seed, float4* XN, float4* NN)
 {
     float z[4];
-    normal4((uint32_t)meta.id(), step, TAG_TILD, 0u, A.seed, z);
+    normal4((uint32_t)meta.id(), step, TAG_TILD, 0u, seed, z);
     const float xcv[3] = {xc.x, xc.y, xc.z};
     float xn[3], nn[3] = {0.f, 0.f, 0.f};
     if (A.integ == MFT_INT_GJF) {
@@ -1345,7 +1393,7 @@ __device__ __forceinline__ int integrate_slot(int s, float4 xc, PMeta meta, cons
         if (A.nz_keyed) {
             // the previous step's nm * normal, the same bits as when it was drawn
             float zo[4];
-            normal4((uint32_t)meta.id(), step - 1u, TAG_TILD, 0u, A.seed, zo);
+            normal4((uint32_t)meta.id(), step - 1u, TAG_TILD, 0u, seed, zo);
             for (int j = 0; j < 3; ++j) nov[j] = nm * zo[j];
         } else {
             nov[0] = nz4.x;
@@ -1397,8 +1445,8 @@ __device__ __forceinline__ int integrate_slot(int s, float4 xc, PMeta meta, cons
             xn[j] = v;
         }
     }
-    ff_store(A.XN, s, xn[0], xn[1], xn[2]);
-    if (A.write_nn) A.NN[s] = make_float4(nn[0], nn[1], nn[2], 0.f);
+    ff_store(XN, s, xn[0], xn[1], xn[2]);
+    if (A.write_nn) NN[s] = make_float4(nn[0], nn[1], nn[2], 0.f);
     return key_of(xn[0], xn[1], xn[2], meta.sp(), A.dx[0], A.dx[1], A.dx[2], A.p, A.nx, A.ny, A.nz, tg);
 }
 
@@ -1407,15 +1455,34 @@ __device__ __forceinline__ int integrate_slot(int s, float4 xc, PMeta meta, cons
 // the slot and counts the next key; integ = MFT_INT_NONE only writes the
 // total force.  TWO: at most two bonds per particle (the slots' bond lists
 // are loaded with the slot's own records, so a slot waits for two rounds of
-// memory latency: its records, then its partners' positions).  dstep: the
-// step index on the device (graph replays), else null.
-template <bool TWO>
+// memory latency: its records, then its partners' positions).
+template <bool TWO, bool BATCH>
 __global__ void __launch_bounds__(256) k_integrate(
     const float4* __restrict__ X, const PMeta* __restrict__ META, const int* __restrict__ BS,
     const int* __restrict__ BT, const float4* __restrict__ fgrid,
     float4* __restrict__ ftot, int maxbonds, BondParams bp, StepArgs A, int ns, int* __restrict__ count,
-    int* __restrict__ key, int* __restrict__ rank, TileGeom tg, const uint32_t* __restrict__ dstep)
+    int* __restrict__ key, int* __restrict__ rank, TileGeom tg, const StepPtrs* __restrict__ tab)
 {
+    // (A itself stays as it came: a changed copy would live in scratch memory)
+    const float4 *XO = A.XO, *NZ = A.NZ;
+    float4 *XN = A.XN, *NN = A.NN;
+    uint64_t seed = A.seed;
+    if constexpr (BATCH) {
+        const auto B = batch_ptrs(tab);
+        X = batch_global(B->X);
+        META = batch_global(B->META);
+        BS = batch_global(B->BS);
+        if (BT) BT = batch_global(B->BT);
+        fgrid = batch_global(B->fgrid);
+        count = batch_global(B->count);
+        key = batch_global(B->key);
+        rank = batch_global(B->rank);
+        XO = batch_global(B->XO);
+        NZ = batch_global(B->NZ);
+        XN = batch_global(B->XN);
+        NN = batch_global(B->NN);
+        seed = B->seed;
+    }
     // contiguous slot ranges per XCD (brick_of_block): bond partners, mostly
     // a few slots away in key order, are read from the L2 that holds the
     // block's own slots rather than from another XCD's lines
@@ -1430,15 +1497,15 @@ __global__ void __launch_bounds__(256) k_integrate(
         const PMeta meta = META[s];
         const bool gjf = A.integ == MFT_INT_GJF;
         const bool need_nz = (gjf && !A.nz_keyed) || A.integ == MFT_INT_VV || A.use_v;
-        const float3 xo3 = gjf ? ff_load(A.XO, s) : make_float3(0.f, 0.f, 0.f);
+        const float3 xo3 = gjf ? ff_load(XO, s) : make_float3(0.f, 0.f, 0.f);
         const float4 xo4 = make_float4(xo3.x, xo3.y, xo3.z, 0.f);
-        const float4 nz4 = need_nz ? A.NZ[s] : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float4 nz4 = need_nz ? NZ[s] : make_float4(0.f, 0.f, 0.f, 0.f);
         int2 bs = make_int2(-1, -1), bt = make_int2(0, 0);
         if constexpr (TWO) {
             bs = reinterpret_cast<const int2*>(BS)[s];
             if (BT) bt = reinterpret_cast<const int2*>(BT)[s];
         }
-        const uint32_t step = dstep ? *dstep : A.step;
+        const uint32_t step = A.step;
         float fo[3] = {fg.x, fg.y, fg.z};
         SpeciesCoef sco;
         if constexpr (TWO) {
@@ -1481,7 +1548,7 @@ __global__ void __launch_bounds__(256) k_integrate(
             langevin_forces(A.lang, meta.id(), meta.sp(), v, A.seed, ls, fo);
         }
         if (ftot) ftot[s] = make_float4(fo[0], fo[1], fo[2], 0.f);
-        if (A.integ != MFT_INT_NONE) k = integrate_slot(s, xc, meta, fo, A, step, tg, xo4, nz4, sco);
+        if (A.integ != MFT_INT_NONE) k = integrate_slot(s, xc, meta, fo, A, step, tg, xo4, nz4, sco, seed, XN, NN);
     }
     if (A.integ == MFT_INT_NONE) return; // uniform over the grid
     const int r = wave_rank(count, k, active);
@@ -1741,32 +1808,39 @@ int tild_unsort(TildEngine* e, int what)
     return MFT_OK;
 }
 
-int tild_scan(TildEngine* e, bool advance_step)
+int tild_scan(TildEngine* e, const TildBatch* b)
 {
-    uint32_t* ds = (advance_step && e->use_dstep) ? e->d_step : nullptr;
+    const StepPtrs* tab = b ? b->tab[e->cur] : nullptr;
+    const unsigned nb = b ? b->n : 1;
     int *count = slot_count(e, e->cur), *other = slot_count(e, 1 - e->cur);
     // what one block of 1024 threads holds is scanned by it alone (8192 keys:
     // 5.4 + 3.7 -> 4.9 us); several such blocks that each read the counts before
     // their own were slower than the reduction's launch (98 304 keys: 13.2 us
     // against 6.1 + 4.4)
     const bool one = e->nkeys <= 1024 * kScanItems;
-    if (!one) k_scan_reduce<<<e->nscan_blocks, kScanThreads, 0, e->stream>>>(count, e->nkeys, e->partial);
-    k_scan_apply<<<one ? 1 : e->nscan_blocks, one ? 1024 : kScanThreads, 0, e->stream>>>(
-        count, other, e->nkeys, e->partial, e->start, e->N, ds);
+    if (!one)
+        (b ? k_scan_reduce<true> : k_scan_reduce<false>)<<<dim3(e->nscan_blocks, 1, nb), kScanThreads, 0, e->stream>>>(
+            count, e->nkeys, e->partial, tab);
+    (b ? k_scan_apply<true> : k_scan_apply<false>)<<<dim3(one ? 1 : e->nscan_blocks, 1, nb),
+                                                     one ? 1024 : kScanThreads, 0, e->stream>>>(
+        count, other, e->nkeys, e->partial, e->start, e->N, tab);
     MFT_LAUNCH_CHECK();
     return MFT_OK;
 }
 
 // next positions into the next key order (after the integrator and the scan)
-int tild_permute(TildEngine* e)
+int tild_permute(TildEngine* e, const TildBatch* b)
 {
     const int N = e->N, mb = std::max(1, e->d.maxbonds), c = e->cur, n = 1 - c;
     // under GJF the next step regenerates the previous noise: NZ stays behind
     const float4* nn = e->d.integrator == MFT_INT_GJF ? nullptr : e->NN;
-    k_permute<<<nblk(N), kBlock, 0, e->stream>>>(N, mb, e->key, e->rank, e->start, e->map, e->XN, nn, e->X[c],
-                                                  e->META[c], slot_bond_types(e, c), e->X[n], e->XO[n], e->NZ[n],
-                                                  e->META[n], slot_bond_types(e, n));
-    k_remap_bonds<<<nblk(N), kBlock, 0, e->stream>>>(N, mb, e->map, e->BS[c], e->BS[n]);
+    const StepPtrs* tab = b ? b->tab[c] : nullptr;
+    const dim3 grid(nblk(N), 1, b ? b->n : 1);
+    (b ? k_permute<true> : k_permute<false>)<<<grid, kBlock, 0, e->stream>>>(
+        N, mb, e->key, e->rank, e->start, e->map, e->XN, nn, e->X[c], e->META[c], slot_bond_types(e, c), e->X[n],
+        e->XO[n], e->NZ[n], e->META[n], slot_bond_types(e, n), tab);
+    (b ? k_remap_bonds<true> : k_remap_bonds<false>)<<<grid, kBlock, 0, e->stream>>>(N, mb, e->map, e->BS[c], e->BS[n],
+                                                                                   tab);
     if (e->d.maxangles > 0)
         k_permute_angles<<<nblk(N), kBlock, 0, e->stream>>>(N, e->d.maxangles, e->map, e->NA[c], e->AT[c], e->AG[c],
                                                             e->NA[n], e->AT[n], e->AG[n]);
@@ -1775,16 +1849,17 @@ int tild_permute(TildEngine* e)
     return MFT_OK;
 }
 
-int tild_density(TildEngine* e)
+int tild_density(TildEngine* e, const TildBatch* b)
 {
     const mft_tild_desc& d = e->d;
     const TileGeom& tg = e->tg;
     const int BM = 1 << tg.lbmax;
     const double inv_gvol = 1.0 / (double)e->gvol;
 #define MFT_DENS(P_, B_)                                                                                  \
-    k_density_tile<P_, B_><<<tg.nbricks, kTileThreads, e->dens_lds, e->stream>>>(                         \
+    (b ? k_density_tile<P_, B_, true> : k_density_tile<P_, B_, false>)<<<                                 \
+        dim3(tg.nbricks, 1, b ? b->n : 1), kTileThreads, e->dens_lds, e->stream>>>(                       \
         e->tiles, e->nchan, e->qchan, e->X[e->cur], e->start, tg, d.nx, d.ny, d.nz, e->dx[0], e->dx[1], \
-        e->dx[2], inv_gvol)
+        e->dx[2], inv_gvol, b ? b->tab[e->cur] : nullptr)
 #define MFT_DENS_B(P_)                                                                                    \
     if (BM == 8) MFT_DENS(P_, 8);                                                                         \
     else MFT_DENS(P_, 4);
@@ -1830,7 +1905,7 @@ bool tild_gather_brick_fits(const TildEngine* e) { return gather_brick_lds(e) <=
 // species), 2 = LDS windows of every species per brick, 3 = as 1 with each
 // workgroup walking a run of (brick, species) tasks, the next window's loads
 // in flight during the current sums
-int tild_gather(TildEngine* e, int mode)
+int tild_gather(TildEngine* e, int mode, const TildBatch* b)
 {
     const mft_tild_desc& d = e->d;
     if (mode == 2 && !tild_gather_brick_fits(e)) mode = 1;
@@ -1917,13 +1992,13 @@ int tild_gather(TildEngine* e, int mode)
         const int BM = 1 << tg.lbmax;
         GatherMap gm;
         for (int sp = 0; sp < kMaxSpecies; ++sp) gm.slot[sp] = sp < d.nspecies ? e->force_slot_h[sp] : -1;
-        dim3 grid(tg.nbricks, d.nspecies);
+        dim3 grid(tg.nbricks, d.nspecies, b ? b->n : 1);
         const float4* Fq = e->F4 + (size_t)(e->qslot >= 0 ? e->qslot : 0) * e->M;
 #define MFT_G1(P_, B_)                                                                                    \
     do {                                                                                                  \
-        k_gather_species<P_, B_><<<grid, kTileThreads, 0, e->stream>>>(e->fgrid, e->F4, gm, e->X[e->cur], e->META[e->cur], \
-                                                                         e->start, tg, d.nx, d.ny, d.nz, e->dx[0], \
-                                                                         e->dx[1], e->dx[2]);             \
+        (b ? k_gather_species<P_, B_, true> : k_gather_species<P_, B_, false>)<<<grid, kTileThreads, 0, e->stream>>>( \
+            e->fgrid, e->F4, gm, e->X[e->cur], e->META[e->cur], e->start, tg, d.nx, d.ny, d.nz, e->dx[0], \
+            e->dx[1], e->dx[2], b ? b->tab[e->cur] : nullptr);                                            \
         if (e->qslot >= 0)                                                                                \
             k_gather_charge<P_, B_><<<tg.nbricks, kTileThreads, 0, e->stream>>>(                          \
                 e->fgrid, Fq, e->X[e->cur], e->META[e->cur], e->start, tg, d.nx, d.ny, d.nz, e->dx[0], e->dx[1], e->dx[2]); \
@@ -1982,24 +2057,17 @@ static StepArgs step_args(const TildEngine* e)
     return A;
 }
 
-int tild_integrate(TildEngine* e, bool want_f)
+int tild_integrate(TildEngine* e, bool want_f, const TildBatch* b)
 {
     const mft_tild_desc& d = e->d;
     const int c = e->cur;
-    const uint32_t* ds = e->use_dstep ? e->d_step : nullptr;
-    if (d.maxbonds == 2)
-        k_integrate<true><<<nblk(e->N), kBlock, 0, e->stream>>>(e->X[c], e->META[c], e->BS[c],
-                                                              slot_bond_types(e, c), e->fgrid,
-                                                              want_f ? e->ftot : nullptr, 2, e->bp,
-                                                              step_args(e), e->N, slot_count(e, c), e->key, e->rank,
-                                                              e->tg,
-                                                              ds);
-    else
-        k_integrate<false><<<nblk(e->N), kBlock, 0, e->stream>>>(e->X[c], e->META[c], e->BS[c],
-                                                               slot_bond_types(e, c), e->fgrid,
-                                                               want_f ? e->ftot : nullptr,
-                                                               std::max(1, d.maxbonds), e->bp, step_args(e), e->N,
-                                                               slot_count(e, c), e->key, e->rank, e->tg, ds);
+    const bool two = d.maxbonds == 2;
+    auto* kernel = b ? (two ? k_integrate<true, true> : k_integrate<false, true>)
+                     : (two ? k_integrate<true, false> : k_integrate<false, false>);
+    kernel<<<dim3(nblk(e->N), 1, b ? b->n : 1), kBlock, 0, e->stream>>>(
+        e->X[c], e->META[c], e->BS[c], slot_bond_types(e, c), e->fgrid, want_f ? e->ftot : nullptr,
+        std::max(1, d.maxbonds), e->bp, step_args(e), e->N, slot_count(e, c), e->key, e->rank, e->tg,
+        b ? b->tab[c] : nullptr);
     MFT_LAUNCH_CHECK();
     return MFT_OK;
 }

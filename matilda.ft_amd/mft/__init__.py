@@ -746,8 +746,8 @@ class FtsSystem:
 
 
 class TildGroup:
-    """Replica group (mft_tild_group_*): engines advanced by one HIP graph of
-    eight steps each; the engines stay owned by the caller."""
+    """Replica group (mft_tild_group_*): engines advanced together, those of one
+    description by shared launches; the engines stay owned by the caller."""
 
     def __init__(self, engines):
         self.engines = list(engines)
