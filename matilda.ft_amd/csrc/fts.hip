@@ -48,6 +48,7 @@ constexpr int kFtsMaxMol = 4;
 constexpr int kFtsMaxBlocks = 16;
 constexpr int kFtsThreads = 256;
 constexpr int kFtsMaxSnapshots = 8;
+constexpr int kFtsSideStreams = 3;
 
 struct FtsPotDev {
     int kind, I, J;
@@ -824,6 +825,9 @@ struct FtsBatch {
     std::deque<FtsRep> reps;
     std::vector<FtsGroup> groups;
     hipStream_t stream = nullptr;
+    // side streams of an iteration's fork and the events around them
+    hipStream_t side[kFtsSideStreams] = {nullptr};
+    hipEvent_t fork = nullptr, join[kFtsSideStreams] = {nullptr};
     int64_t* d_iter = nullptr;       // iteration counter per slot
     int nslots = 0;
     std::vector<int> free_slots;
@@ -1456,10 +1460,9 @@ static int launch_prop_xy(const PropDesc* dx, const PropDesc* dy, int n, const F
 }
 
 // propagators, densities and Q of every replica in the group
-static int group_density(FtsBatch* b, FtsGroup& G)
+static int group_density(FtsBatch* b, FtsGroup& G, hipStream_t st)
 {
     int rc;
-    hipStream_t st = b->stream;
     const bool fused = plane_fused(G) && b->plane_xy;
     for (const auto& chunk : G.bead_at)
         for (int s = 0; s < (int)chunk.size(); ++s)
@@ -1520,22 +1523,22 @@ __global__ void __launch_bounds__(256) k_fts_zero_mean(const ZmDesc* __restrict_
     D.w[i] = make_float2((float)((double)w.x - mx), (float)((double)w.y - my));
 }
 
-static int group_update(FtsBatch* b, FtsGroup& G, int first);
+static int group_update(FtsBatch* b, FtsGroup& G, int first, hipStream_t st);
 
 // zero-mean fields (after a correction only the EMPC ones), then the species
 // fields, E and the H sums again
-static int group_zero_mean(FtsBatch* b, FtsGroup& G, bool corrector)
+static int group_zero_mean(FtsBatch* b, FtsGroup& G, bool corrector, hipStream_t st)
 {
     const int n = corrector ? G.nzm_pc : G.nzm;
     if (!n) return MFT_OK;
     const int M = G.n[0] * G.n[1] * G.n[2];
     dim3 grid((M + 255) / 256, n);
-    k_fts_zero_mean<<<grid, 256, 0, b->stream>>>(G.d_zm);
+    k_fts_zero_mean<<<grid, 256, 0, st>>>(G.d_zm);
     MFT_LAUNCH_CHECK();
-    return group_update(b, G, 1);
+    return group_update(b, G, 1, st);
 }
 
-static int group_update(FtsBatch* b, FtsGroup& G, int first)
+static int group_update(FtsBatch* b, FtsGroup& G, int first, hipStream_t st)
 {
     const int M = G.n[0] * G.n[1] * G.n[2];
     const int nr = (int)G.reps.size();
@@ -1548,7 +1551,7 @@ static int group_update(FtsBatch* b, FtsGroup& G, int first)
     dim3 grid((M + kFtsThreads - 1) / kFtsThreads, nr);
     const FtsUpdDev* d = G.d_upd + (size_t)first * nr;
 #define MFT_UPD(S_, P_)                                                                                   \
-    if (NS == S_ && NP == P_) k_fts_update<S_, P_><<<grid, kFtsThreads, 0, b->stream>>>(d);
+    if (NS == S_ && NP == P_) k_fts_update<S_, P_><<<grid, kFtsThreads, 0, st>>>(d);
     MFT_UPD(2, 2) MFT_UPD(2, 4) MFT_UPD(2, 8) MFT_UPD(4, 2) MFT_UPD(4, 4) MFT_UPD(4, 8) MFT_UPD(8, 2)
     MFT_UPD(8, 4) MFT_UPD(8, 8)
 #undef MFT_UPD
@@ -1655,8 +1658,8 @@ static int batch_activate(FtsBatch* b, const std::vector<int>& reps)
     for (auto& kv : tmp) {
         FtsGroup& T = kv.second;
         if (!rc) rc = group_setup(b, T);
-        if (!rc) rc = group_update(b, T, 1);
-        if (!rc) rc = group_density(b, T);
+        if (!rc) rc = group_update(b, T, 1, b->stream);
+        if (!rc) rc = group_density(b, T, b->stream);
     }
     // the temporary descriptors are read by the launches just queued
     hipError_t e = hipStreamSynchronize(b->stream);
@@ -1733,6 +1736,11 @@ static int batch_destroy(FtsBatch* b)
     for (auto& r : b->reps) free_all(r.allocs);
     for (auto& G : b->groups) free_all(G.allocs);
     free_all(b->allocs);
+    for (hipStream_t st : b->side)
+        if (st) (void)hipStreamDestroy(st);
+    for (hipEvent_t ev : b->join)
+        if (ev) (void)hipEventDestroy(ev);
+    if (b->fork) (void)hipEventDestroy(b->fork);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
     return MFT_OK;
@@ -1750,8 +1758,8 @@ static int batch_init(FtsBatch* b)
     for (auto& G : b->groups) {
         if (G.reps.empty()) continue;
         if ((rc = group_ready(b, G))) return rc;
-        if ((rc = group_update(b, G, 1))) return rc;
-        if ((rc = group_density(b, G))) return rc;
+        if ((rc = group_update(b, G, 1, b->stream))) return rc;
+        if ((rc = group_density(b, G, b->stream))) return rc;
     }
     b->inited = true;
     return MFT_OK;
@@ -1790,10 +1798,9 @@ static int fft3(float2* a, const FtsRep& r, int sign, hipStream_t st)
 
 // the k-space step of every 1S field of the group (forces from the pass just
 // run): w <- IFFT[(w_k - dt (F_k - A w_k)) / (1 + dt A)]
-static int group_one_step(FtsBatch* b, FtsGroup& G)
+static int group_one_step(FtsBatch* b, FtsGroup& G, hipStream_t st)
 {
     int rc;
-    hipStream_t st = b->stream;
     for (int id : G.reps) {
         FtsRep& r = b->reps[id];
         for (int p = 0; p < r.d.npotentials; ++p) {
@@ -1818,28 +1825,67 @@ static int group_one_step(FtsBatch* b, FtsGroup& G)
     return MFT_OK;
 }
 
-// one CL iteration of every group: field updates from the previous
-// densities, propagators, densities and Q; then every slot's counter
-// advances (a slot is reset when a replica takes it)
+// one CL iteration of a group: field updates from the previous densities,
+// propagators, densities and Q
+static int group_iteration(FtsBatch* b, FtsGroup& G, hipStream_t st)
+{
+    int rc;
+    if ((rc = group_update(b, G, 0, st))) return rc;
+    if (G.s1) {
+        // k-space step of the 1S fields, then the species fields again
+        if ((rc = group_one_step(b, G, st))) return rc;
+        if ((rc = group_update(b, G, 1, st))) return rc;
+    }
+    if ((rc = group_zero_mean(b, G, false, st))) return rc;
+    if ((rc = group_density(b, G, st))) return rc;
+    if (G.pc) {
+        // FTS_Box.cu:53-81: correct, rebuild species fields, densities again
+        if ((rc = group_update(b, G, 2, st))) return rc;
+        if ((rc = group_zero_mean(b, G, true, st))) return rc;
+        if ((rc = group_density(b, G, st))) return rc;
+    }
+    return MFT_OK;
+}
+
+// stream k of a fork: the batch's own, then up to three of its side streams
+// (made on first use; four hardware queues serve a process)
+static int side_stream(FtsBatch* b, int k, hipStream_t* st)
+{
+    *st = b->stream;
+    if (k == 0) return MFT_OK;
+    if (!b->fork) MFT_HIP(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
+    if (!b->side[k - 1]) MFT_HIP(hipStreamCreateWithFlags(&b->side[k - 1], hipStreamNonBlocking));
+    if (!b->join[k - 1]) MFT_HIP(hipEventCreateWithFlags(&b->join[k - 1], hipEventDisableTiming));
+    *st = b->side[k - 1];
+    return MFT_OK;
+}
+
+// One CL iteration of every group, then every slot's counter advances (a slot is
+// reset when a replica takes it).  A group's beads are a chain of dependent
+// launches of a few microseconds that fills the chip only with many replicas, and
+// groups share nothing within an iteration, so they run side by side on up to
+// four streams (uneven replicas on four grids, us an iteration: 4 replicas 1611 ->
+// 1017, 16 replicas 3670 -> 2097, 64 replicas 9093 -> 7862).
 static int batch_iteration(FtsBatch* b)
 {
     int rc;
-    for (auto& G : b->groups) {
-        if (G.reps.empty()) continue;
-        if ((rc = group_update(b, G, 0))) return rc;
-        if (G.s1) {
-            // k-space step of the 1S fields, then the species fields again
-            if ((rc = group_one_step(b, G))) return rc;
-            if ((rc = group_update(b, G, 1))) return rc;
-        }
-        if ((rc = group_zero_mean(b, G, false))) return rc;
-        if ((rc = group_density(b, G))) return rc;
-        if (G.pc) {
-            // FTS_Box.cu:53-81: correct, rebuild species fields, densities again
-            if ((rc = group_update(b, G, 2))) return rc;
-            if ((rc = group_zero_mean(b, G, true))) return rc;
-            if ((rc = group_density(b, G))) return rc;
-        }
+    std::vector<FtsGroup*> groups;
+    for (auto& G : b->groups)
+        if (!G.reps.empty()) groups.push_back(&G);
+    const int nst = std::min((int)groups.size(), kFtsSideStreams + 1);
+    for (int k = 1; k < nst; ++k) {
+        hipStream_t st;
+        if ((rc = side_stream(b, k, &st))) return rc;
+        if (k == 1) MFT_HIP(hipEventRecord(b->fork, b->stream));
+        MFT_HIP(hipStreamWaitEvent(st, b->fork, 0));
+    }
+    for (size_t g = 0; g < groups.size(); ++g) {
+        hipStream_t st;
+        if ((rc = side_stream(b, (int)g % nst, &st)) || (rc = group_iteration(b, *groups[g], st))) return rc;
+    }
+    for (int k = 1; k < nst; ++k) {
+        MFT_HIP(hipEventRecord(b->join[k - 1], b->side[k - 1]));
+        MFT_HIP(hipStreamWaitEvent(b->stream, b->join[k - 1], 0));
     }
     for (int o = 0; o < b->nslots; o += 256) {
         int cnt = std::min(256, b->nslots - o);
@@ -2347,9 +2393,9 @@ int mft_fts_batch_autotune(mft_fts_batch* b, int reps, double* ms_per_pass)
         for (size_t c : cand) {
             if (c != 0 && c >= ws) continue;   // one chunk anyway
             G.chunk_bytes = c;
-            if ((rc = group_setup(b, G)) || (rc = group_density(b, G))) break;   // warm
+            if ((rc = group_setup(b, G)) || (rc = group_density(b, G, b->stream))) break;   // warm
             MFT_HIP(hipEventRecord(e0, b->stream));
-            for (int r = 0; r < reps && !rc; ++r) rc = group_density(b, G);
+            for (int r = 0; r < reps && !rc; ++r) rc = group_density(b, G, b->stream);
             if (rc) break;
             MFT_HIP(hipEventRecord(e1, b->stream));
             MFT_HIP(hipEventSynchronize(e1));
