@@ -184,7 +184,8 @@ MFT_PLAN_LOW(160, 16, 2, 2, 2, 2, 2, 5)
 MFT_PLAN_LOW(256, 64, 4, 4, 4, 4)
 #undef MFT_PLAN_LOW
 
-// Plans of the particle-mesh engine's x and y passes: the default but where it
+// Plans of single-line passes (the transform plan, the particle-mesh engine's x and
+// y passes): the default but where it
 // holds 12 or 20 elements a thread, which serialises a line over two or four
 // threads (24^3, two channels: x pass from the density tiles
 // 11.5 -> 6.5 us, last inverse x pass 7.8 -> 5.4 us).
