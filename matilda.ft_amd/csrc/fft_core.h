@@ -185,12 +185,21 @@ MFT_PLAN_LOW(256, 64, 4, 4, 4, 4)
 #undef MFT_PLAN_LOW
 
 // Plans of single-line passes (the transform plan, the particle-mesh engine's x and
-// y passes): the default but where it
-// holds 12 or 20 elements a thread, which serialises a line over two or four
-// threads (24^3, two channels: x pass from the density tiles
-// 11.5 -> 6.5 us, last inverse x pass 7.8 -> 5.4 us).
+// y passes): the default, but more threads and fewer elements where it holds 12 or
+// 20 elements a thread, which serialises a line over one to eight threads (24^3,
+// last inverse x pass 7.8 -> 5.4 us), and up to 32 points, where a small grid's
+// lines would not fill the chip (32^3 4.5 -> 3.8 us).  At 64 points four elements
+// a thread change nothing and at 128 the y pass slows from 28 to 45 us.
 template <int N>
-struct FftPlanMesh : std::conditional_t<(FftPlan<N>::E > 8 && N > 12), FftPlanLow<N>, FftPlan<N>> {};
+struct FftPlanMesh
+    : std::conditional_t<(FftPlan<N>::E > (N <= 32 ? 4 : 8) && N > 12), FftPlanLow<N>, FftPlan<N>> {};
+
+// Plans of the forward x pass that sums the density tiles: a thread sums as many
+// points, of up to eight tile entries each, as it holds elements of the line, so
+// this pass takes few elements at every length (24^3 11.5 -> 6.5 us, 32^3 6.8 ->
+// 4.7, 64^3 with three channels 11.3 -> 8.7, 128^3 37 -> 33).
+template <int N>
+struct FftPlanTiles : std::conditional_t<(FftPlan<N>::E > 4 && N > 12), FftPlanLow<N>, FftPlan<N>> {};
 
 // Expands F(N) for every supported size; used by host dispatch switches.
 #define MFT_FOR_EACH_FFT_SIZE(F)                                                 \

@@ -124,7 +124,7 @@ __global__ void __launch_bounds__(256) k_fft_x_fwd_tiles(const float* __restrict
         tiles = batch_global(batch_ptrs(btab)->tiles);
         out = batch_global(batch_ptrs(btab)->S);
     }
-    using P = FftPlanMesh<N>;
+    using P = FftPlanTiles<N>;
     constexpr int T = P::T, E = P::E, B = 256 / T;
     constexpr int NP = swz_pitch(N);
     __shared__ float2 lds[B * NP];
@@ -529,7 +529,7 @@ __global__ void __launch_bounds__(256) k_fft_x_fwd_tiles_staged(const float* __r
                                                                 long cstride, int ex0,
                                                                 const float2* __restrict__ twg)
 {
-    using P = FftPlanMesh<N>;
+    using P = FftPlanTiles<N>;
     constexpr int T = P::T, E = P::E, B = 256 / T;
     extern __shared__ float4 stage4[];   // [2 z covers][B lines][2 y covers][ex0 / 4]
     float* stage = reinterpret_cast<float*>(stage4);
@@ -612,7 +612,7 @@ __global__ void __launch_bounds__(256) k_fft_x_fwd_tiles_staged(const float* __r
 bool tild_x_fwd_staged_ok(int nx, int ex0, int maxcover)
 {
     int T = 0;
-#define MFT_T(n_) if (nx == n_) T = FftPlanMesh<n_>::T;
+#define MFT_T(n_) if (nx == n_) T = FftPlanTiles<n_>::T;
     MFT_FOR_EACH_FFT_SIZE(MFT_T)
 #undef MFT_T
     if (T == 0 || ex0 % 4 != 0 || maxcover > 2) return false;
@@ -627,7 +627,7 @@ int tild_x_fwd_tiles(const float* tiles, const int* tab, float2* S, int nx, int 
         switch (nx) {
 #define MFT_CASE(n_)                                                                                      \
     case n_: {                                                                                            \
-        constexpr int B = 256 / FftPlanMesh<n_>::T;                                                           \
+        constexpr int B = 256 / FftPlanTiles<n_>::T;                                                           \
         dim3 grid((ny * nz + B - 1) / B, nchan);                                                          \
         k_fft_x_fwd_tiles_staged<n_><<<grid, 256, 16 * B * (size_t)ex0, st>>>(tiles, tab, S, ny, nz, cstride, ex0, \
                                                                             fft_twiddles_device(n_));    \
@@ -643,7 +643,7 @@ int tild_x_fwd_tiles(const float* tiles, const int* tab, float2* S, int nx, int 
     switch (nx) {
 #define MFT_CASE(n_)                                                                                      \
     case n_: {                                                                                            \
-        constexpr int B = 256 / FftPlanMesh<n_>::T;                                                           \
+        constexpr int B = 256 / FftPlanTiles<n_>::T;                                                           \
         dim3 grid((ny * nz + B - 1) / B, nchan, nbatch);                                                  \
         constexpr bool many = n_ <= kBatchMaxGrid;                                                        \
         (btab && many ? k_fft_x_fwd_tiles<n_, many> : k_fft_x_fwd_tiles<n_>)<<<grid, 256, 0, st>>>(       \
