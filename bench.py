@@ -200,7 +200,7 @@ def tild_c1_measure(steps=200, replicas=16, seed=1234):
     """The plain TILD diblock melt (2000 chains of 10 A + 10 B, 40 000
     particles, 20^3 box, 32^3 grid, GJF): stepped alone, as a one-replica
     graph group (two steps per graph launch), and as a group of `replicas`
-    such systems (different seeds) advanced by one graph; particle-steps/s
+    such systems (different seeds) advanced together; particle-steps/s
     over all replicas."""
     import mft
     from mft import systems
