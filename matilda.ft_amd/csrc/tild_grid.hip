@@ -297,21 +297,33 @@ __global__ void __launch_bounds__(256) k_fft_x_fwd_tiles(const float* __restrict
 // The x and y transforms of one z-plane of an N x N grid in one workgroup:
 // the plane sits in LDS with a row pitch of N + 1 (a column's elements fall in
 // different banks) and its lines are transformed in place, T consecutive
-// threads per line (so a line's exchanges stay inside one wavefront), LINES
-// lines at a time.  The arithmetic is that of the line passes (same plans,
-// twiddles and summation order; the compiler may still contract different
-// multiply-adds in the two kernels, so results can differ by rounding); the
-// plane passes save one HBM round trip of the spectra per direction.
+// threads per line (so a line's exchanges stay inside one wavefront), as many
+// lines at a time as the workgroup has threads for.  The arithmetic is that of
+// the line passes: each direction takes the plan of the pass it replaces (rows
+// of the forward direction FftPlanTiles, the others FftPlanMesh), with the same
+// twiddles and summation order, so that a choice between the two forms does not
+// change the plan; the compiler may still contract different multiply-adds in
+// the two kernels, so results can differ by rounding.  The plane passes save one
+// HBM round trip of the spectra per direction.
+constexpr int plane_lines(int n, int t) // the most lines of n that divide n and take at most 1024 threads
+{
+    int l = n;
+    while (n % l || l * t > 1024) --l;
+    return l;
+}
+
 template <int N>
 struct PlaneShape {
-    using P = FftPlan<N>;
+    using P = FftPlanMesh<N>;
+    using PX = FftPlanTiles<N>;
     static constexpr int T = P::T, E = P::E;
-    static constexpr int NT = T * N >= 1024 ? 1024 : T * N;
-    static constexpr int LINES = NT / T;
+    static constexpr int LINES = plane_lines(N, T);
+    static constexpr int NT = LINES * T;
     static constexpr int ROUNDS = N / LINES;
+    static constexpr int TX = PX::T, EX = PX::E, LINESX = NT / TX;
     static constexpr int PITCH = N + 1;
     static constexpr size_t LDS = sizeof(float2) * N * PITCH;
-    static_assert(N % LINES == 0, "whole rounds of lines");
+    static_assert(NT % 64 == 0 && NT % TX == 0 && N % LINESX == 0, "whole wavefronts and whole rounds of rows");
 };
 
 // Forward x then y transforms of channel blockIdx.y, z-plane blockIdx.x, from
@@ -338,25 +350,27 @@ __global__ void __launch_bounds__(PlaneShape<N>::NT) k_fft_xy_fwd_tiles_plane(
         plane[y * PITCH + x] = make_float2(tile_sum(tc, tz, tabxy + 5 * (N + y), tabxy + 5 * x), 0.f);
     }
     __syncthreads();
-    const int lt = threadIdx.x / T, t = threadIdx.x % T;
+    constexpr int TX = S::TX, EX = S::EX, LINESX = S::LINESX;
 #pragma unroll
-    for (int r = 0; r < S::ROUNDS; ++r) {
-        LdsMap map{r * LINES + lt, 0, false, PITCH};   // row y
-        float2 v[E];
+    for (int r = 0; r < N / LINESX; ++r) {
+        const int lt = threadIdx.x / TX, t = threadIdx.x % TX;
+        LdsMap map{r * LINESX + lt, 0, false, PITCH};   // row y
+        float2 v[EX];
 #pragma unroll
-        for (int s = 0; s < E; ++s) v[s] = plane[map(t + T * s)];
-        line_fft<N, -1, true>(v, plane, tw, t, map);
+        for (int s = 0; s < EX; ++s) v[s] = plane[map(t + TX * s)];
+        line_fft_plan<typename S::PX, -1, true>(v, plane, tw, t, map);
 #pragma unroll
-        for (int s = 0; s < E; ++s) plane[map(t + T * s)] = v[s];
+        for (int s = 0; s < EX; ++s) plane[map(t + TX * s)] = v[s];
     }
     __syncthreads();
+    const int lt = threadIdx.x / T, t = threadIdx.x % T;
 #pragma unroll
     for (int r = 0; r < S::ROUNDS; ++r) {
         LdsMap map{r * LINES + lt, PITCH, true, N};    // column x
         float2 v[E];
 #pragma unroll
         for (int s = 0; s < E; ++s) v[s] = plane[map(t + T * s)];
-        line_fft<N, -1, true>(v, plane, tw, t, map);
+        line_fft_plan<typename S::P, -1, true>(v, plane, tw, t, map);
 #pragma unroll
         for (int s = 0; s < E; ++s) plane[map(t + T * s)] = v[s];
     }
@@ -414,7 +428,7 @@ __global__ void __launch_bounds__(PlaneShape<N>::NT) k_fft_yx_inv_packed_plane(
                 float2 v[E];
 #pragma unroll
                 for (int s = 0; s < E; ++s) v[s] = plane[map(t + T * s)];
-                line_fft<N, +1, true>(v, plane, tw, t, map);
+                line_fft_plan<typename S::P, +1, true>(v, plane, tw, t, map);
 #pragma unroll
                 for (int s = 0; s < E; ++s) plane[map(t + T * s)] = v[s];
             }
@@ -428,7 +442,7 @@ __global__ void __launch_bounds__(PlaneShape<N>::NT) k_fft_yx_inv_packed_plane(
                 LdsMap map{row, 0, false, PITCH};          // row y
 #pragma unroll
                 for (int s = 0; s < E; ++s) v[s] = plane[map(t + T * s)];
-                line_fft<N, +1, true>(v, plane, tw, t, map);
+                line_fft_plan<typename S::P, +1, true>(v, plane, tw, t, map);
             } else {
 #pragma unroll
                 for (int s = 0; s < E; ++s) v[s] = make_float2(0.f, 0.f);
