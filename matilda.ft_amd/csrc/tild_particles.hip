@@ -10,7 +10,10 @@ namespace mft {
 // bound by that: consecutive lanes take consecutive entries of one particle's
 // row.  A thread that walked a whole row alone touched 64 cache lines per load
 // (164 k particles, p = 3, two species: weights 386 us, density 2 x 254, forces
-// 2 x 410; now 17, 2 x 81 and 2 x 33, the weights at 5.0 TB/s of writes).
+// 2 x 410; now 17, 2 x 81 and 2 x 33, the weights at 5.0 TB/s of writes).  With
+// several threads per particle a call can need more threads than a launch takes
+// (2^32), so the kernels walk their work in strides of the grid.
+static unsigned table_blocks(long n) { return (unsigned)std::min((n + 255) / 256, 1L << 23); }
 
 // ------------------------------------------------- grid weights (T3) ----
 constexpr int kWeightParticles = 32; // particles per workgroup
@@ -22,30 +25,32 @@ __global__ void __launch_bounds__(256) k_grid_weights(float* __restrict__ W, int
 {
     __shared__ float w[kWeightParticles][3][p + 1];
     __shared__ int g[kWeightParticles][3][p + 1]; // the stencil's offsets into the grid, per axis
-    const int first = blockIdx.x * kWeightParticles;
-    const int np = min(kWeightParticles, ns - first);
-    if ((int)threadIdx.x < 3 * np) {
-        const int i = threadIdx.x / 3, j = threadIdx.x - 3 * i;
-        const float dx = j == 0 ? dx0 : (j == 1 ? dx1 : dx2);
-        const int n = j == 0 ? nx : (j == 1 ? ny : nz), pitch = j == 0 ? 1 : (j == 1 ? nx : nx * ny);
-        float wj[5];
-        const int base = base_index_weights(x[(long)(first + i) * 3 + j], dx, p, wj) - p / 2;
-#pragma unroll
-        for (int k = 0; k <= p; ++k) {
-            w[i][j][k] = wj[k];
-            g[i][j][k] = (base + k + n) % n * pitch;
-        }
-    }
-    __syncthreads();
     // the device kernel divides by the float product of the float spacings
     const float gvol = dx0 * dx1 * dx2;
     constexpr int p1 = p + 1, G = p1 * p1 * p1;
-    const long o0 = (long)first * G;
-    for (int k = threadIdx.x; k < np * G; k += 256) {
-        const int i = k / G, e = k - i * G;
-        const int ix = e / (p1 * p1), r = e - ix * p1 * p1, iy = r / p1, iz = r - iy * p1;
-        inds[o0 + k] = g[i][0][ix] + g[i][1][iy] + g[i][2][iz];
-        W[o0 + k] = w[i][0][ix] * w[i][1][iy] * w[i][2][iz] / gvol;
+    for (long first = (long)blockIdx.x * kWeightParticles; first < ns; first += (long)gridDim.x * kWeightParticles) {
+        const int np = (int)min((long)kWeightParticles, ns - first);
+        if ((int)threadIdx.x < 3 * np) {
+            const int i = threadIdx.x / 3, j = threadIdx.x - 3 * i;
+            const float dx = j == 0 ? dx0 : (j == 1 ? dx1 : dx2);
+            const int n = j == 0 ? nx : (j == 1 ? ny : nz), pitch = j == 0 ? 1 : (j == 1 ? nx : nx * ny);
+            float wj[5];
+            const int base = base_index_weights(x[(first + i) * 3 + j], dx, p, wj) - p / 2;
+#pragma unroll
+            for (int k = 0; k <= p; ++k) {
+                w[i][j][k] = wj[k];
+                g[i][j][k] = (base + k + n) % n * pitch;
+            }
+        }
+        __syncthreads();
+        const long o0 = first * G;
+        for (int k = threadIdx.x; k < np * G; k += 256) {
+            const int i = k / G, e = k - i * G;
+            const int ix = e / (p1 * p1), r = e - ix * p1 * p1, iy = r / p1, iz = r - iy * p1;
+            inds[o0 + k] = g[i][0][ix] + g[i][1][iy] + g[i][2][iz];
+            W[o0 + k] = w[i][0][ix] * w[i][1][iy] * w[i][2][iz] / gvol;
+        }
+        __syncthreads(); // the next particles' stencils take these ones' place
     }
 }
 
@@ -61,16 +66,16 @@ __global__ void __launch_bounds__(256) k_fill_density_tables(unsigned long long*
                                                              const int* __restrict__ inds,
                                                              const float* __restrict__ W, int G, int M, int ns)
 {
-    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nentries) return;
-    const int s = (int)(k / G), p = sites[s];
-    if (p < 0 || p >= ns) return;
-    const long o = (long)p * G + (k - (long)s * G);
-    const int gi = inds[o];
-    if (gi < 0 || gi >= M) return;
-    const float w = W[o];
-    atomicAdd(&acc[gi], (unsigned long long)__float2ll_rn(w * 4294967296.0f));
-    if (accq) atomicAdd(&accq[gi], (unsigned long long)__float2ll_rn(w * q[p] * 4294967296.0f));
+    for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < nentries; k += (long)gridDim.x * blockDim.x) {
+        const int s = (int)(k / G), p = sites[s];
+        if (p < 0 || p >= ns) continue;
+        const long o = (long)p * G + (k - (long)s * G);
+        const int gi = inds[o];
+        if (gi < 0 || gi >= M) continue;
+        const float w = W[o];
+        atomicAdd(&acc[gi], (unsigned long long)__float2ll_rn(w * 4294967296.0f));
+        if (accq) atomicAdd(&accq[gi], (unsigned long long)__float2ll_rn(w * q[p] * 4294967296.0f));
+    }
 }
 
 __global__ void k_fixed_to_float_add(float* __restrict__ out, const unsigned long long* __restrict__ acc, int M)
@@ -91,29 +96,32 @@ __global__ void __launch_bounds__(256) k_map_forces_tables(float* __restrict__ f
                                                            const float* __restrict__ W, int G, float gvol, int M,
                                                            int ns)
 {
-    const int s = (int)(((long)blockIdx.x * blockDim.x + threadIdx.x) / kMapLanes);
+    constexpr int kSites = 256 / kMapLanes; // sites of a workgroup at a time
     const int lane = threadIdx.x % kMapLanes;
-    const int p = s < nsites ? sites[s] : -1;
-    const bool valid = p >= 0 && p < ns;
-    float a[3] = {0.f, 0.f, 0.f};
-    if (valid) {
-        const long o = (long)p * G;
-        for (int i = lane; i < G; i += kMapLanes) {
-            const int gi = inds[o + i];
-            if (gi < 0 || gi >= M) continue;
-            const float w = W[o + i] * gvol;
-            const float* F = gridF + (long)gi * 3;
+    for (long first = (long)blockIdx.x * kSites; first < nsites; first += (long)gridDim.x * kSites) {
+        const long s = first + threadIdx.x / kMapLanes;
+        const int p = s < nsites ? sites[s] : -1;
+        const bool valid = p >= 0 && p < ns;
+        float a[3] = {0.f, 0.f, 0.f};
+        if (valid) {
+            const long o = (long)p * G;
+            for (int i = lane; i < G; i += kMapLanes) {
+                const int gi = inds[o + i];
+                if (gi < 0 || gi >= M) continue;
+                const float w = W[o + i] * gvol;
+                const float* F = gridF + (long)gi * 3;
 #pragma unroll
-            for (int j = 0; j < 3; ++j) a[j] = fmaf(F[j], w, a[j]);
+                for (int j = 0; j < 3; ++j) a[j] = fmaf(F[j], w, a[j]);
+            }
         }
+#pragma unroll
+        for (int h = 1; h < kMapLanes; h <<= 1)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) a[j] += __shfl_xor(a[j], h, kMapLanes);
+        if (!valid || lane >= 3) continue;
+        const float v = lane == 0 ? a[0] : (lane == 1 ? a[1] : a[2]);
+        f[(long)p * 3 + lane] += q ? v * q[p] : v;
     }
-#pragma unroll
-    for (int h = 1; h < kMapLanes; h <<= 1)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) a[j] += __shfl_xor(a[j], h, kMapLanes);
-    if (!valid || lane >= 3) return;
-    const float v = lane == 0 ? a[0] : (lane == 1 ? a[1] : a[2]);
-    f[(long)p * 3 + lane] += q ? v * q[p] : v;
 }
 
 // ----------------------------------------------------------- bonds ------
@@ -2185,7 +2193,7 @@ int mft_tild_grid_weights(float* gridW, int* gridInds, const float* x, int ns, c
     MFT_REQUIRE(gridW && gridInds && x && Nx && dx && ns >= 0, MFT_ERR_INVALID, "null argument");
     MFT_REQUIRE(pmeorder >= 0 && pmeorder <= 4, MFT_ERR_INVALID, "pmeorder must be 0..4");
     if (ns == 0) return MFT_OK;
-    const unsigned blocks = (ns + kWeightParticles - 1) / kWeightParticles;
+    const unsigned blocks = table_blocks((long)ns * (256 / kWeightParticles));
     switch (pmeorder) {
 #define MFT_CASE(p_)                                                                                      \
     case p_:                                                                                              \
@@ -2209,16 +2217,21 @@ int mft_tild_fill_density(float* rho, float* rhoq, const float* q, const int* si
     unsigned long long* acc = nullptr;
     int rc;
     if ((rc = dalloc(&acc, (size_t)M * (rhoq ? 2 : 1)))) return rc;
-    MFT_HIP(hipMemsetAsync(acc, 0, sizeof(unsigned long long) * (size_t)M * (rhoq ? 2 : 1), st));
-    if (nsites > 0)
-        k_fill_density_tables<<<nblk((long)nsites * G), kBlock, 0, st>>>(
-            acc, rhoq ? acc + M : nullptr, q, sites, (long)nsites * G, gridInds, gridW, G, M, ns);
-    k_fixed_to_float_add<<<nblk(M), kBlock, 0, st>>>(rho, acc, M);
-    if (rhoq) k_fixed_to_float_add<<<nblk(M), kBlock, 0, st>>>(rhoq, acc + M, M);
-    MFT_LAUNCH_CHECK();
-    MFT_HIP(hipStreamSynchronize(st));
-    MFT_HIP(hipFree(acc));
-    return MFT_OK;
+    auto run = [&]() -> int {
+        MFT_HIP(hipMemsetAsync(acc, 0, sizeof(unsigned long long) * (size_t)M * (rhoq ? 2 : 1), st));
+        if (nsites > 0)
+            k_fill_density_tables<<<table_blocks((long)nsites * G), 256, 0, st>>>(
+                acc, rhoq ? acc + M : nullptr, q, sites, (long)nsites * G, gridInds, gridW, G, M, ns);
+        k_fixed_to_float_add<<<nblk(M), kBlock, 0, st>>>(rho, acc, M);
+        if (rhoq) k_fixed_to_float_add<<<nblk(M), kBlock, 0, st>>>(rhoq, acc + M, M);
+        MFT_LAUNCH_CHECK();
+        MFT_HIP(hipStreamSynchronize(st));
+        return MFT_OK;
+    };
+    rc = run();
+    const hipError_t err = hipFree(acc); // waits for whatever run() queued
+    if (!rc) MFT_HIP(err);
+    return rc;
 }
 
 int mft_tild_map_forces(float* f, const float* gridF, const float* q, const int* sites, int nsites, int ns,
@@ -2226,7 +2239,7 @@ int mft_tild_map_forces(float* f, const float* gridF, const float* q, const int*
 {
     MFT_REQUIRE(f && gridF && sites && gridInds && gridW && nsites >= 0 && G > 0, MFT_ERR_INVALID, "null argument");
     if (nsites == 0) return MFT_OK;
-    k_map_forces_tables<<<nblk((long)nsites * kMapLanes), kBlock, 0, (hipStream_t)stream>>>(
+    k_map_forces_tables<<<table_blocks((long)nsites * kMapLanes), 256, 0, (hipStream_t)stream>>>(
         f, gridF, q, sites, nsites, gridInds, gridW, G, gvol, M, ns);
     MFT_LAUNCH_CHECK();
     return MFT_OK;

@@ -69,3 +69,44 @@ def test_pair_force_of_a_table_without_symmetry(gpu, grid):
         e = rel(got[:, j], F0[:, j] + 1.7 * V.real.reshape(-1))
         say("pair force", grid, j, "%.2e" % e)
         assert e < 2e-6
+
+
+def test_calls_of_more_threads_than_a_launch_takes(gpu):
+    """A launch takes fewer than 2^32 threads.  2^28 + 2000 sites at 16 lanes a site (force map) or 64 entries a
+    site (density), nearly all of them empty, and the weights of 2^29 + 37 particles at eight threads each."""
+    n, ns, G, Nx = 2 ** 28 + 2000, 700, 64, (12, 10, 16)
+    M = int(np.prod(Nx))
+    rng = np.random.default_rng(5)
+    L = np.array([4.0, 3.0, 5.0], np.float32)
+    dx = (L / np.array(Nx, np.float32)).astype(np.float32)
+    x = (rng.random((ns, 3)) * L).astype(np.float32)
+    inds, W = gpu.grid_weights(x.reshape(-1), Nx, dx, 3)
+    F = rng.normal(size=(M, 3)).astype(np.float32)
+    own = np.concatenate([np.arange(300), n - 1 - np.arange(300), 2 ** 26 - 50 + np.arange(100)])
+    sites = np.full(n, -1, np.int32)
+    sites[own] = np.arange(ns, dtype=np.int32)
+    few = np.arange(ns, dtype=np.int32)
+    say("case: table calls past 2^32 threads")
+    assert np.array_equal(gpu.fill_density(M, sites, inds, W, G)[0], gpu.fill_density(M, few, inds, W, G)[0])
+    assert np.array_equal(gpu.map_forces(ns, F.reshape(-1), sites, inds, W, G, 0.1),
+                          gpu.map_forces(ns, F.reshape(-1), few, inds, W, G, 0.1))
+    del sites
+    # order 0: one entry a particle; all at the origin but some at either side of a sweep of the grid
+    n = 2 ** 29 + 37
+    at = np.array([0, 31, 2 ** 28 - 1, 2 ** 28, 2 ** 28 + 33, n - 2, n - 1])
+    xd, Wd, Id = gpu.DeviceBuffer(12 * n), gpu.DeviceBuffer(4 * n), gpu.DeviceBuffer(4 * n)
+    xd.zero()
+    for k, i in enumerate(at):
+        gpu.check(gpu.lib().mft_memcpy_h2d(ctypes.c_void_p(xd.ptr.value + 12 * int(i)),
+                                           x[k].ctypes.data_as(ctypes.c_void_p), ctypes.c_size_t(12)))
+    gpu.check(gpu.lib().mft_tild_grid_weights(Wd.ptr, Id.ptr, xd.ptr, n, (ctypes.c_int * 3)(*Nx),
+                                              (ctypes.c_float * 3)(*dx), 0, None))
+    want, wantW = gpu.grid_weights(x[: at.size].reshape(-1), Nx, dx, 0)
+    got = Id.to_array(np.int32, (n,))
+    assert np.array_equal(got[at], want)
+    got[at] = 0
+    assert not got.any()
+    got = Wd.to_array(np.float32, (n,))
+    assert np.array_equal(got[at], wantW) and np.all(got == wantW[0])
+    for b in (xd, Wd, Id):
+        b.free()
