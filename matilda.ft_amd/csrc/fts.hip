@@ -29,6 +29,7 @@
 
 #include "common.h"
 #include "fft_core.h"
+#include "fork_join.h"
 #include "fts_bead.h"
 
 namespace mft {
@@ -1731,7 +1732,10 @@ static void graph_drop(FtsBatch* b);
 static int batch_destroy(FtsBatch* b)
 {
     if (!b) return MFT_OK;
+    // the side streams too: a join that failed left one unordered
     if (b->stream) (void)hipStreamSynchronize(b->stream);
+    for (hipStream_t st : b->side)
+        if (st) (void)hipStreamSynchronize(st);
     graph_drop(b);
     for (auto& r : b->reps) free_all(r.allocs);
     for (auto& G : b->groups) free_all(G.allocs);
@@ -1847,12 +1851,10 @@ static int group_iteration(FtsBatch* b, FtsGroup& G, hipStream_t st)
     return MFT_OK;
 }
 
-// stream k of a fork: the batch's own, then up to three of its side streams
-// (made on first use; four hardware queues serve a process)
+// side stream k >= 1 of a fork, with its events (made on first use; four hardware
+// queues serve a process: the batch's own stream and up to three of these)
 static int side_stream(FtsBatch* b, int k, hipStream_t* st)
 {
-    *st = b->stream;
-    if (k == 0) return MFT_OK;
     if (!b->fork) MFT_HIP(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
     if (!b->side[k - 1]) MFT_HIP(hipStreamCreateWithFlags(&b->side[k - 1], hipStreamNonBlocking));
     if (!b->join[k - 1]) MFT_HIP(hipEventCreateWithFlags(&b->join[k - 1], hipEventDisableTiming));
@@ -1872,21 +1874,24 @@ static int batch_iteration(FtsBatch* b)
     std::vector<FtsGroup*> groups;
     for (auto& G : b->groups)
         if (!G.reps.empty()) groups.push_back(&G);
-    const int nst = std::min((int)groups.size(), kFtsSideStreams + 1);
-    for (int k = 1; k < nst; ++k) {
-        hipStream_t st;
-        if ((rc = side_stream(b, k, &st))) return rc;
-        if (k == 1) MFT_HIP(hipEventRecord(b->fork, b->stream));
-        MFT_HIP(hipStreamWaitEvent(st, b->fork, 0));
-    }
-    for (size_t g = 0; g < groups.size(); ++g) {
-        hipStream_t st;
-        if ((rc = side_stream(b, (int)g % nst, &st)) || (rc = group_iteration(b, *groups[g], st))) return rc;
-    }
-    for (int k = 1; k < nst; ++k) {
-        MFT_HIP(hipEventRecord(b->join[k - 1], b->side[k - 1]));
-        MFT_HIP(hipStreamWaitEvent(b->stream, b->join[k - 1], 0));
-    }
+    const int n = (int)groups.size();
+    rc = fork_join(
+        std::min(n, kFtsSideStreams + 1), n,
+        [&](int k) -> int {
+            hipStream_t st;
+            const int r = side_stream(b, k, &st);
+            if (r) return r;
+            if (k == 1) MFT_HIP(hipEventRecord(b->fork, b->stream));
+            MFT_HIP(hipStreamWaitEvent(st, b->fork, 0));
+            return MFT_OK;
+        },
+        [&](int g, int k) -> int { return group_iteration(b, *groups[g], k ? b->side[k - 1] : b->stream); },
+        [&](int k) -> int {
+            MFT_HIP(hipEventRecord(b->join[k - 1], b->side[k - 1]));
+            MFT_HIP(hipStreamWaitEvent(b->stream, b->join[k - 1], 0));
+            return MFT_OK;
+        });
+    if (rc) return rc;
     for (int o = 0; o < b->nslots; o += 256) {
         int cnt = std::min(256, b->nslots - o);
         k_fts_iter_incr<<<1, 256, 0, b->stream>>>(b->d_iter + o, cnt);
