@@ -974,9 +974,21 @@ int mft_fts_propagate(float* q, float* qdag, const float* W, const float* g, con
         }
         return st;
     };
-    const long apart = nchains == 2 ? out[1] - out[0] : 0; // the chains as two fields of one array
     const float scale = (float)(1.0 / (double)M);
     const AxisGeom gx{Nx[0], Nx[1], Nx[2], 0}, gy{Nx[0], Nx[1], Nx[2], 1};
+    // a line pass over both chains: two fields of one array, or, where their
+    // distance is no whole number of points (float arrays are 4-byte aligned),
+    // a launch each
+    const long bytes = nchains == 2 ? (char*)out[1] - (char*)out[0] : 0, apart = bytes / (long)sizeof(float2);
+    const bool together = bytes % (long)sizeof(float2) == 0;
+    auto axis = [&](int sign, float2* (*in)(const ChainStep&), float2* (*to)(const ChainStep&), const ChainSteps& cs,
+                    AxisGeom geom, float sc) {
+        int r = tild_axis(sign, 0, 0, in(cs.c[0]), to(cs.c[0]), geom, together ? nchains : 1, apart, sc, st);
+        if (!r && !together) r = tild_axis(sign, 0, 0, in(cs.c[1]), to(cs.c[1]), geom, 1, 0, sc, st);
+        return r;
+    };
+    float2* (*const slot)(const ChainStep&) = [](const ChainStep& C) { return C.slot; };
+    float2* (*const next)(const ChainStep&) = [](const ChainStep& C) { return C.next; };
     const bool planes = chain_plane(ChainSteps{}, 0, Nx, false, scale, st, true) == MFT_OK;
     for (int s = 0; s < Ntot; ++s) {
         const ChainSteps cs = steps(s);
@@ -985,7 +997,7 @@ int mft_fts_propagate(float* q, float* qdag, const float* W, const float* g, con
         } else if (s == 0) {
             k_chain_first<<<dim3(nblk(M), nchains), 256, 0, st>>>(cs, M);
         } else {
-            if ((rc = tild_axis(+1, 0, 0, cs.c[0].slot, cs.c[0].slot, gy, nchains, apart, 1.0f, st))) return rc;
+            if ((rc = axis(+1, slot, slot, cs, gy, 1.0f))) return rc;
             switch (Nx[0]) {
 #define MFT_CASE(n_) case n_: launch_chain_x<n_>(cs, nchains, Nx[1] * Nx[2], st); break;
                 MFT_FOR_EACH_FFT_SIZE(MFT_CASE)
@@ -994,8 +1006,8 @@ int mft_fts_propagate(float* q, float* qdag, const float* W, const float* g, con
         }
         if (s + 1 == Ntot) break;
         if (!planes) {
-            if ((rc = tild_axis(-1, 0, 0, cs.c[0].slot, cs.c[0].next, gx, nchains, apart, scale, st))) return rc;
-            if ((rc = tild_axis(-1, 0, 0, cs.c[0].next, cs.c[0].next, gy, nchains, apart, 1.0f, st))) return rc;
+            if ((rc = axis(-1, slot, next, cs, gx, scale))) return rc;
+            if ((rc = axis(-1, next, next, cs, gy, 1.0f))) return rc;
         }
         switch (Nx[2]) {
 #define MFT_CASE(n_) case n_: launch_chain_z<n_>(cs, nchains, (const float2*)g, Nx[0] * Nx[1], st); break;

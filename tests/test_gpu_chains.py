@@ -55,3 +55,23 @@ def test_propagate_matches_numpy(gpu, grid, blocks, want):
         e = rel(got[c], np.array(ref))
         say("propagate", grid, blocks, want, c, "%.2e" % e)
         assert e < 3e-6
+
+
+@pytest.mark.parametrize("grid", [(20, 20, 2), (12, 12, 8), (16, 20, 24), (6, 96, 10)])
+def test_chains_an_odd_number_of_floats_apart(gpu, grid):
+    """The arrays are floats to the caller: a complementary chain that starts at any float of an allocation gives the
+    bits it gives at an aligned address, on grids of either form."""
+    rng = np.random.default_rng(sum(grid))
+    M, n = int(np.prod(grid)), 5
+    W = ((rng.normal(size=(2, M)) + 1j * rng.normal(size=(2, M))) * 0.2).astype(np.complex64)
+    g = np.exp(-rng.random(M)).astype(np.complex64)
+    want = chains(gpu, W, g, ((2, 0), (3, 1)), grid, "qd")
+    mol = gpu.FtsMoleculeC()
+    mol.nblocks = 2
+    mol.N[0], mol.species[0], mol.N[1], mol.species[1] = 2, 0, 3, 1
+    Wb, gb = gpu.DeviceBuffer.from_array(W), gpu.DeviceBuffer.from_array(g)
+    q, qd = gpu.DeviceBuffer(8 * M * n), gpu.DeviceBuffer(8 * M * n + 4)
+    gpu.check(gpu.lib().mft_fts_propagate(q.ptr, ctypes.c_void_p(qd.ptr.value + 4), Wb.ptr, gb.ptr, ctypes.byref(mol),
+                                          (ctypes.c_int * 3)(*grid), None))
+    assert np.array_equal(q.to_array(np.complex64, (n, M)), want[0])
+    assert np.array_equal(qd.to_array(np.float32, 2 * M * n + 1)[1:].view(np.complex64).reshape(n, M), want[1])
