@@ -958,10 +958,12 @@ int mft_fts_propagate(float* q, float* qdag, const float* W, const float* g, con
     float2* out[2] = {nullptr, nullptr};
     if (q && q != qdag) out[nchains] = (float2*)q, which[nchains++] = 0;
     if (qdag) out[nchains] = (float2*)qdag, which[nchains++] = 1;
-    std::vector<int> species;
-    for (int b = 0; b < mol->nblocks; ++b) species.insert(species.end(), mol->N[b], mol->species[b]);
-    Ntot = (int)species.size();
-    auto spec = [&](int c, int s) { return species[which[c] == 0 ? s : Ntot - 1 - s]; };
+    for (int b = 0; b < mol->nblocks; ++b) Ntot += mol->N[b];
+    auto spec = [&](int c, int s) {
+        int at = which[c] == 0 ? s : Ntot - 1 - s, b = 0;
+        while (at >= mol->N[b]) at -= mol->N[b++];
+        return mol->species[b];
+    };
     auto steps = [&](int s) {
         ChainSteps st = {};
         for (int c = 0; c < nchains; ++c) {
