@@ -34,15 +34,17 @@ const float2* fft_twiddles_device(int n)
     return d;
 }
 
-// Lines of 20, 40, 48, 80, 96 points take plans of at most ten elements a thread
-// (FftPlanMesh; forward and back, 96 x 80 x 64 batch of 4 63.3 -> 60.6 us,
-// 40 x 48 x 32 29.7 -> 24.7 us): with 12 or 20 a line runs on one to eight threads.
+// Lines of 16, 20, 24, 40, 48, 80, 96 and 160 points take plans of at most ten
+// elements a thread (FftPlanLines; one direction, with the default plans -> now: 24^3
+// x 4 14.6 -> 10.5 us, 48^3 x 4 17.2 -> 15.4, 40 x 48 x 32 14.7 -> 11.3, 96 x 80 x 64 x 4
+// 35.3 -> 32.6, 160 x 160 x 40 x 2 42.2 -> 37.5): with 12 or 20 elements a line runs on
+// one to eight threads.
 template <int N, int SIGN>
 __global__ void __launch_bounds__(256) k_fft_lines(const float2* __restrict__ in, float2* __restrict__ out,
                                                    AxisGeom geom, long field_stride, const float2* __restrict__ twg,
                                                    float scale)
 {
-    using P = FftPlanMesh<N>;
+    using P = FftPlanLines<N>;
     constexpr int T = P::T, E = P::E, B = 256 / T;
     __shared__ float2 lds[B * N];
     __shared__ float2 tw[N];
@@ -74,7 +76,7 @@ static int launch_lines(const float2* in, float2* out, AxisGeom g, int batch, lo
     switch (g.length()) {
 #define MFT_CASE(n_)                                                                                       \
     case n_: {                                                                                             \
-        constexpr int B = 256 / FftPlanMesh<n_>::T;                                                          \
+        constexpr int B = 256 / FftPlanLines<n_>::T;                                                          \
         dim3 grid((g.nlines() + B - 1) / B, batch);                                                        \
         k_fft_lines<n_, SIGN><<<grid, 256, 0, st>>>(in, out, g, fs, fft_twiddles_device(n_), scale);       \
         break;                                                                                             \

@@ -119,6 +119,36 @@ struct Dft<5, SIGN> {
     }
 };
 
+// Twice an odd length R / 2 = H, by the prime-factor mapping: input n = H n1 + 2 n2,
+// output k = k1 mod 2, k2 mod H, so that the parts need no twiddles between them
+// (as separate levels they round once more at most outputs).
+template <int R, int SIGN>
+__device__ __forceinline__ void dft_even_odd(float2* a)
+{
+    constexpr int H = R / 2;
+    float2 s[H], d[H];
+#pragma unroll
+    for (int n = 0; n < H; ++n) {
+        s[n] = cadd(a[2 * n], a[(2 * n + H) % R]);
+        d[n] = csub(a[2 * n], a[(2 * n + H) % R]);
+    }
+    Dft<H, SIGN>::run(s);
+    Dft<H, SIGN>::run(d);
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+        a[k % 2 ? k + H : k] = s[k]; // the even index that is k mod H
+        a[k % 2 ? k : k + H] = d[k]; // the odd one
+    }
+}
+template <int SIGN>
+struct Dft<6, SIGN> {
+    __device__ __forceinline__ static void run(float2* a) { dft_even_odd<6, SIGN>(a); }
+};
+template <int SIGN>
+struct Dft<10, SIGN> {
+    __device__ __forceinline__ static void run(float2* a) { dft_even_odd<10, SIGN>(a); }
+};
+
 // ------------------------------------------------------------ plans ------
 template <int... Rs>
 struct Radices {};
@@ -184,20 +214,48 @@ MFT_PLAN_LOW(160, 16, 2, 2, 2, 2, 2, 5)
 MFT_PLAN_LOW(256, 64, 4, 4, 4, 4)
 #undef MFT_PLAN_LOW
 
-// Plans of single-line passes (the transform plan, the particle-mesh engine's x and
-// y passes): the default, but more threads and fewer elements where it holds 12 or
-// 20 elements a thread, which serialises a line over one to eight threads (24^3,
-// last inverse x pass 7.8 -> 5.4 us), and up to 32 points, where a small grid's
-// lines would not fill the chip (32^3 4.5 -> 3.8 us).  At 64 points four elements
-// a thread change nothing and at 128 the y pass slows from 28 to 45 us.
+// Plans of the particle-mesh engine's x and y passes: the default, but more threads
+// and fewer elements where it holds 12 or 20 elements a thread, which serialises a
+// line over one to eight threads (24^3, last inverse x pass 7.8 -> 5.4 us), and up to
+// 32 points, where a small grid's lines would not fill the chip (32^3 4.5 -> 3.8 us).
+// At 64 points four elements a thread change nothing and at 128 the y pass slows from
+// 28 to 45 us.  192 points keep 12 elements: no plan of fewer is built for them.
 template <int N>
 struct FftPlanMesh
     : std::conditional_t<(FftPlan<N>::E > (N <= 32 ? 4 : 8) && N > 12), FftPlanLow<N>, FftPlan<N>> {};
 
+// Plans of the transform plan (mft_fft_exec): at most ten elements a thread at the
+// lengths that are no power of two, and four at 16 points, with the odd radix and a
+// factor of two as one level.  As separate levels of radix 2 the transforms rounded
+// more often than with the default plans: random lines forward / back, 1e-8 (default;
+// separate levels; these): 48 points 8.08 / 8.04; 8.21 / 8.25; 7.94 / 7.73, 80 points
+// 8.98 / 8.48; 9.09 / 8.64; 8.92 / 8.31, 96 points 8.95 / 9.01; 9.08 / 9.36; 8.78 /
+// 8.86, 160 points 9.65 / 9.42; 9.78 / 9.59; 9.51 / 9.16.  32 points keep 8 x 4, which
+// errs least (7.16, against 7.40 with 4 x 4 x 2 and 7.24 with 2 x 4 x 4).
+template <int N>
+struct FftPlanLines : FftPlan<N> {};
+#define MFT_PLAN_LINES(N_, T_, ...)                                             \
+    template <>                                                                 \
+    struct FftPlanLines<N_> {                                                   \
+        static constexpr int N = N_;                                            \
+        static constexpr int T = T_;                                            \
+        static constexpr int E = N_ / T_;                                       \
+        using R = Radices<__VA_ARGS__>;                                         \
+    };
+MFT_PLAN_LINES(16, 4, 4, 4)
+MFT_PLAN_LINES(20, 2, 2, 10)
+MFT_PLAN_LINES(24, 4, 6, 2, 2)
+MFT_PLAN_LINES(40, 4, 2, 2, 10)
+MFT_PLAN_LINES(48, 8, 2, 2, 2, 6)
+MFT_PLAN_LINES(80, 8, 2, 2, 2, 10)
+MFT_PLAN_LINES(96, 16, 2, 2, 2, 2, 6)
+MFT_PLAN_LINES(160, 16, 2, 2, 2, 2, 10)
+#undef MFT_PLAN_LINES
+
 // Plans of the forward x pass that sums the density tiles: a thread sums as many
 // points, of up to eight tile entries each, as it holds elements of the line, so
-// this pass takes few elements at every length (24^3 11.5 -> 6.5 us, 32^3 6.8 ->
-// 4.7, 64^3 with three channels 11.3 -> 8.7, 128^3 37 -> 33).
+// this pass takes few elements at every length that has such a plan (24^3 11.5 -> 6.5
+// us, 32^3 6.8 -> 4.7, 64^3 with three channels 11.3 -> 8.7, 128^3 37 -> 33).
 template <int N>
 struct FftPlanTiles : std::conditional_t<(FftPlan<N>::E > 4 && N > 12), FftPlanLow<N>, FftPlan<N>> {};
 
