@@ -45,6 +45,51 @@ __global__ void k_real_to_complex(float2* __restrict__ out, const float* __restr
     if (i < M) out[i] = make_float2(in[i], 0.f);
 }
 
+// A level of the density: the mean of 64 of its points, spread over the grid, the
+// same bits in every wavefront.
+__device__ __forceinline__ float rho_level(const float* __restrict__ rho, long M)
+{
+    float c = rho[(long)(threadIdx.x & 63) * M / 64];
+#pragma unroll
+    for (int h = 1; h < 64; h <<= 1) c += __shfl_xor(c, h);
+    return c * (1.0f / 64.0f);
+}
+
+// Forward pass along x of the density less its level (whose force k_pair_x adds).
+// A density is far from zero mean and a transform rounds relative to all of it;
+// components 0 and 1 of the force share a transform below, so the rounding of one's
+// imaginary part, which a transform each would discard, is in the other's real part.
+// Without the mean the force errs less than with a transform each (two-species melt,
+// gaussian table, error against 64 bits of a transform each; shared; shared without
+// the mean: 64^3 2.27e-7; 2.40e-7; 1.89e-7, 96^3 2.46e-7; 2.62e-7; 2.25e-7).
+template <int N>
+__global__ void __launch_bounds__(256) k_pair_rho(float2* __restrict__ S, const float* __restrict__ rho, int nlines,
+                                                  float scale, const float2* __restrict__ twg)
+{
+    using P = FftPlan<N>;
+    constexpr int T = P::T, E = P::E, B = 256 / T;
+    __shared__ float2 lds[B * N];
+    __shared__ float2 tw[N];
+    for (int i = threadIdx.x; i < N; i += 256) tw[i] = twg[i];
+    const int lline = threadIdx.x / T, t = threadIdx.x % T;
+    const int line = blockIdx.x * B + lline;
+    const bool valid = line < nlines;
+    const long base = (long)line * N + t;
+    float r[E];
+#pragma unroll
+    for (int s = 0; s < E; ++s) r[s] = valid ? rho[base + T * s] : 0.f;
+    const float level = rho_level(rho, (long)N * nlines);
+    float2 v[E];
+#pragma unroll
+    for (int s = 0; s < E; ++s) v[s] = make_float2(r[s] - level, 0.f);
+    __syncthreads();
+    LdsMap map{lline, B, false, N};
+    line_fft<N, -1>(v, lds, tw, t, map);
+    if (!valid) return;
+#pragma unroll
+    for (int s = 0; s < E; ++s) S[base + T * s] = cscale(v[s], scale);
+}
+
 // Pair force along z: forward transform of the density's spectrum S (x and y
 // done), the three products with fk, inverse transforms.  Only the real part of
 // each force component is kept, which is the transform of the Hermitian part of
@@ -100,12 +145,14 @@ __global__ void __launch_bounds__(256) k_pair_z(float2* __restrict__ S, float2* 
     }
 }
 
-// Last inverse pass along x of both fields, added to the force grid:
+// Last inverse pass along x of both fields, added to the force grid with the force
+// of the level (that of a constant density: none in any table of a potential):
 // gridF[i*3 + j] += factor * component j (accumulateGridForceComp,
 // ps_groups.cu:164-178)
 template <int N>
 __global__ void __launch_bounds__(256) k_pair_x(float* __restrict__ gridF, const float2* __restrict__ P01,
-                                                const float2* __restrict__ P2, int nlines, float factor,
+                                                const float2* __restrict__ P2, const float* __restrict__ rho,
+                                                const float2* __restrict__ fk, int nlines, float factor,
                                                 const float2* __restrict__ twg)
 {
     using P = FftPlan<N>;
@@ -123,6 +170,8 @@ __global__ void __launch_bounds__(256) k_pair_x(float* __restrict__ gridF, const
         u[s] = valid ? P01[base + T * s] : make_float2(0.f, 0.f);
         v[s] = valid ? P2[base + T * s] : make_float2(0.f, 0.f);
     }
+    const float level = rho_level(rho, (long)N * nlines);
+    const float f0 = level * fk[0].x, f1 = level * fk[1].x, f2 = level * fk[2].x;
     __syncthreads();
     LdsMap map{lline, B, false, N};
     line_fft<N, +1>(u, lds, tw, t, map);
@@ -131,9 +180,9 @@ __global__ void __launch_bounds__(256) k_pair_x(float* __restrict__ gridF, const
 #pragma unroll
     for (int s = 0; s < E; ++s) {
         float* F = gridF + 3 * (base + T * s);
-        F[0] = fmaf(factor, u[s].x, F[0]);
-        F[1] = fmaf(factor, u[s].y, F[1]);
-        F[2] = fmaf(factor, v[s].x, F[2]);
+        F[0] = fmaf(factor, u[s].x + f0, F[0]);
+        F[1] = fmaf(factor, u[s].y + f1, F[1]);
+        F[2] = fmaf(factor, v[s].x + f2, F[2]);
     }
 }
 
@@ -145,10 +194,18 @@ static void launch_pair_z(float2* S, float2* P01, const float2* fk, int nx, int 
 }
 
 template <int N>
-static void launch_pair_x(float* gridF, const float2* P01, const float2* P2, int nlines, float factor, hipStream_t st)
+static void launch_pair_rho(float2* S, const float* rho, int nlines, float scale, hipStream_t st)
 {
     constexpr int B = 256 / FftPlan<N>::T;
-    k_pair_x<N><<<(nlines + B - 1) / B, 256, 0, st>>>(gridF, P01, P2, nlines, factor, fft_twiddles_device(N));
+    k_pair_rho<N><<<(nlines + B - 1) / B, 256, 0, st>>>(S, rho, nlines, scale, fft_twiddles_device(N));
+}
+
+template <int N>
+static void launch_pair_x(float* gridF, const float2* P01, const float2* P2, const float* rho, const float2* fk,
+                          int nlines, float factor, hipStream_t st)
+{
+    constexpr int B = 256 / FftPlan<N>::T;
+    k_pair_x<N><<<(nlines + B - 1) / B, 256, 0, st>>>(gridF, P01, P2, rho, fk, nlines, factor, fft_twiddles_device(N));
 }
 
 __global__ void k_mul_inplace(float2* __restrict__ a, const float2* __restrict__ b, long M)
@@ -245,8 +302,12 @@ int mft_tild_pair_force(float* gridF, const float* rho, const float* fk, const i
     float2* S = (float2*)work;
     float2* P01 = S + M;
     const int nx = Nx[0], ny = Nx[1], nz = Nx[2];
-    const AxisGeom gx{nx, ny, nz, 0}, gy{nx, ny, nz, 1};
-    if ((rc = tild_axis(-1, 1, 0, rho, S, gx, 1, M, (float)(1.0 / (double)M), st))) return rc;
+    const AxisGeom gy{nx, ny, nz, 1};
+    switch (nx) {
+#define MFT_CASE(n_) case n_: launch_pair_rho<n_>(S, rho, ny * nz, (float)(1.0 / (double)M), st); break;
+        MFT_FOR_EACH_FFT_SIZE(MFT_CASE)
+#undef MFT_CASE
+    }
     if ((rc = tild_axis(-1, 0, 0, S, S, gy, 1, M, 1.0f, st))) return rc;
     switch (nz) {
 #define MFT_CASE(n_) case n_: launch_pair_z<n_>(S, P01, (const float2*)fk, nx, ny, st); break;
@@ -255,7 +316,7 @@ int mft_tild_pair_force(float* gridF, const float* rho, const float* fk, const i
     }
     if ((rc = tild_axis(+1, 0, 0, S, S, gy, 2, M, 1.0f, st))) return rc;
     switch (nx) {
-#define MFT_CASE(n_) case n_: launch_pair_x<n_>(gridF, P01, S, ny * nz, factor, st); break;
+#define MFT_CASE(n_) case n_: launch_pair_x<n_>(gridF, P01, S, rho, (const float2*)fk, ny * nz, factor, st); break;
         MFT_FOR_EACH_FFT_SIZE(MFT_CASE)
 #undef MFT_CASE
     }

@@ -696,12 +696,10 @@ static int launch_axis(const void* in, void* out, AxisGeom g, int nf, long fs, f
     return MFT_OK;
 }
 
-// the three variants in use: forward real -> complex, forward and inverse
-// complex -> complex
+// the two variants in use: forward and inverse complex -> complex
 int tild_axis(int sign, int real_in, int real_out, const void* in, void* out, AxisGeom g, int nf, long fs,
               float scale, hipStream_t st)
 {
-    if (sign < 0 && real_in && !real_out) return launch_axis<FftPlan, -1, true, false>(in, out, g, nf, fs, scale, st);
     if (sign < 0 && !real_in && !real_out) return launch_axis<FftPlan, -1, false, false>(in, out, g, nf, fs, scale, st);
     if (sign > 0 && !real_in && !real_out) return launch_axis<FftPlan, +1, false, false>(in, out, g, nf, fs, scale, st);
     set_error(MFT_ERR_UNSUPPORTED, "axis pass variant not built");

@@ -110,3 +110,21 @@ def test_calls_of_more_threads_than_a_launch_takes(gpu):
     assert np.array_equal(got[at], wantW) and np.all(got == wantW[0])
     for b in (xd, Wd, Id):
         b.free()
+
+
+@pytest.mark.parametrize("grid", [(16, 20, 24), (64, 48, 12), (12, 12, 96)])
+def test_pair_force_of_a_density_far_from_zero_mean(gpu, grid):
+    """The transforms round relative to the density's fluctuations, not to its mean: the bound of the table without
+    symmetry holds for a mean of 200 fluctuations, whose rounding alone would be 200 times 1e-7."""
+    rng = np.random.default_rng(sum(grid))
+    M, sh = int(np.prod(grid)), grid[::-1]
+    rho = (200.0 + rng.normal(size=M)).astype(np.float32)
+    k = np.meshgrid(*[2 * np.pi * np.fft.fftfreq(n) for n in sh], indexing="ij")
+    u = np.exp(-sum(a * a for a in k))
+    fk = np.stack([-1j * a * u for a in k[::-1]], -1).reshape(M, 3).astype(np.complex64)
+    got = gpu.pair_force(np.zeros(3 * M, np.float32), rho, fk, grid, factor=1.0).reshape(M, 3)
+    S = np.fft.fftn((rho.astype(np.float64) - 200.0).reshape(sh))
+    want = np.stack([np.fft.ifftn(fk[:, j].reshape(sh) * S).real.reshape(-1) for j in range(3)], -1)
+    e = rel(got, want)
+    say("pair force, mean of 200", grid, "%.2e" % e)
+    assert e < 2e-6
