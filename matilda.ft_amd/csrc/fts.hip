@@ -1099,6 +1099,9 @@ static int rep_setup(FtsBatch* b, FtsRep& r)
     }
     if (b->plane_xy && bead_grid(ns)) {
         for (int a = 0; a < 3; ++a) {
+            for (int e = 0; e < a; ++e) // an axis like an earlier one shares its table
+                if (ns[e] == ns[a] && Ls[e] == Ls[a]) r.bt[a] = r.bt[e];
+            if (r.bt[a]) continue;
             std::vector<double> g(ns[a]);
             for (int i = 0; i < ns[a]; ++i) g[i] = axis_factor(i, ns[a], Ls[a], d.Nr);
             std::vector<float> tab;
