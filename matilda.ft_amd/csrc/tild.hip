@@ -1,6 +1,7 @@
 // TILD engine: set-up, channel layout, the step loop and the C entry points
 // of the engine (mft_tild_create .. mft_tild_autotune).  Kernels live in
 // tild_particles.hip, tild_grid.hip and tild_conv.hip.
+#include "fork_join.h"
 #include "tild_impl.h"
 
 namespace mft {
@@ -1307,20 +1308,28 @@ int mft_tild_group_step(mft_tild_group* g, int nsteps)
         MFT_HIP(hipMemcpy(g->table, want.data(), sizeof(StepPtrs) * want.size(), hipMemcpyHostToDevice));
         g->uploaded = want;
     }
-    // a lead's stream runs after the work its members already have on theirs
+    // a lead's stream runs after the work its members already have on theirs, and
+    // theirs after it, also where a launch fails in between
     size_t first = 0;
     for (const auto& b : batches) {
         if (b.size() > 1) {
             std::vector<TildEngine*> eng;
             for (int i : b) eng.push_back(g->eng[i]);
-            for (size_t k = 1; k < b.size(); ++k) {
-                MFT_HIP(hipEventRecord(g->ev[b[k]], eng[k]->stream));
-                MFT_HIP(hipStreamWaitEvent(eng[0]->stream, g->ev[b[k]], 0));
-            }
             const TildBatch tb{{g->table + first, g->table + n + first}, (int)b.size()};
-            if ((rc = batch_steps(eng, tb, nsteps))) return rc;
-            MFT_HIP(hipEventRecord(g->ev[b[0]], eng[0]->stream));
-            for (size_t k = 1; k < b.size(); ++k) MFT_HIP(hipStreamWaitEvent(eng[k]->stream, g->ev[b[0]], 0));
+            rc = fork_join(
+                (int)b.size(), 1,
+                [&](int k) -> int {
+                    MFT_HIP(hipEventRecord(g->ev[b[k]], eng[k]->stream));
+                    MFT_HIP(hipStreamWaitEvent(eng[0]->stream, g->ev[b[k]], 0));
+                    return MFT_OK;
+                },
+                [&](int, int) { return batch_steps(eng, tb, nsteps); },
+                [&](int k) -> int {
+                    if (k == 1) MFT_HIP(hipEventRecord(g->ev[b[0]], eng[0]->stream));
+                    MFT_HIP(hipStreamWaitEvent(eng[k]->stream, g->ev[b[0]], 0));
+                    return MFT_OK;
+                });
+            if (rc) return rc;
         }
         first += b.size();
     }
