@@ -328,8 +328,9 @@ int mft_tild_set_grid_passes(mft_tild* eng, int variant);
  * step on their own streams.  Each engine gives the same bits as when stepped
  * alone.  To share launches engines need GJF or EM, no grid line over 64 points,
  * the default gather and grid passes, one charge per species, no ramps, bias,
- * walls, angles, DPD or Langevin potentials, and timing off.  The engines stay
- * owned by the caller; destroy the group before them. */
+ * walls, angles, DPD or Langevin potentials, and timing off; up to three boxes
+ * over 48 points step on their own streams.  The engines stay owned by the
+ * caller; destroy the group before them. */
 typedef struct mft_tild_group mft_tild_group;
 int mft_tild_group_create(mft_tild_group** grp, mft_tild* const* engines, int n);
 int mft_tild_group_destroy(mft_tild_group* grp);

@@ -1249,7 +1249,26 @@ static std::vector<std::vector<int>> group_batches(const mft_tild_group* g)
             }
         if (!joined) out.push_back({i});
     }
-    return out;
+    // Two or three boxes over 48 points that are alone on their streams fill the chip
+    // and overlap better there: 64^3 with 225 k particles, us a step of all, shared ->
+    // own streams: two 129 -> 117, three 165 -> 148, but four 202 -> 244 and eight 358 ->
+    // 421 (four hardware queues serve a process); 48^3, two 104 -> 100, four 142 -> 202.
+    auto large = [&](const std::vector<int>& b) {
+        const mft_tild_desc& d = g->eng[b[0]]->d;
+        return std::max(d.nx, std::max(d.ny, d.nz)) > 48;
+    };
+    size_t own = 0;
+    for (const auto& b : out)
+        if (b.size() == 1 || large(b)) own += b.size();
+    if (own > 3) return out;
+    std::vector<std::vector<int>> split;
+    for (const auto& b : out) {
+        if (large(b))
+            for (int i : b) split.push_back({i});
+        else
+            split.push_back(b);
+    }
+    return split;
 }
 
 extern "C" {

@@ -58,3 +58,63 @@ def test_batched_replicas_equal_engines_alone(gpu, grid, box, pme, integrator, c
     grp.close()
     for e in alone + grouped:
         e.close()
+
+
+@pytest.mark.parametrize("counts", [(2,), (3,), (4,), (2, 1), (2, 3)])
+def test_two_or_three_large_boxes_and_more(gpu, counts):
+    """Up to three boxes over 48 points that would be alone on their streams step there, more of them or small ones
+    share launches: either way the bits of each engine alone."""
+    cfgs = []
+    for k, n in enumerate(counts):  # the first description 64 points, the second 24
+        cfgs += [systems.tild_diblock(nchains=120 - 20 * k, NA=5, NB=6, box=(14.0, 8.0)[k], grid=(64, 24)[k],
+                                      seed=10 * k + r) for r in range(n)]
+    alone, grouped = ([systems.tild_engine(c, "GJF") for c in cfgs] for _ in range(2))
+    grp = gpu.TildGroup(grouped)
+    for n in (1, 3, 2):
+        for e in alone:
+            e.step(n)
+        grp.step(n)
+    for a, b in zip(alone, grouped):
+        for u, v in zip(state(a), state(b)):
+            assert np.array_equal(u, v), counts
+    grp.close()
+    for e in alone + grouped:
+        e.close()
+
+
+def engine(cfg, integrator, bonds):
+    t = cfg["topo"]
+    import mft
+    e = mft.TildEngine(cfg["Nx"], cfg["L"], cfg["pmeorder"], len(cfg["species"]), t["type"].size, cfg["potentials"],
+                       bonds["k"], bonds["r0"], bonds["style"], integrator=integrator, delt=cfg["delt"],
+                       mass=cfg["mass"], mobility=cfg["mobility"], seed=cfg["seed"])
+    e.set_topology(t["type"], None, t["nBonds"], t["bondedTo"], t["bondType"])
+    e.set_state(cfg["x"])
+    return e
+
+
+@pytest.mark.parametrize("grid, box, style, erf", [(24, 9.0, 0, True), (20, 8.0, 1, True), (40, 13.0, 1, False),
+                                                   (48, 15.0, 0, True)])
+def test_batched_tables_bond_kinds_and_scan_sizes(gpu, grid, box, style, erf):
+    """Shared launches with potentials that are tables, two bond types, FENE bonds (style 1), and key counts on either
+    side of what one workgroup scans (16 384: 40^3 in bricks of 8 has 16 000, 48^3 27 648)."""
+    cfgs = []
+    for seed in range(4):
+        c = systems.tild_diblock(nchains=150, NA=5, NB=6, box=box, grid=grid, seed=40 + seed)
+        c["topo"]["bondType"] = (np.arange(c["topo"]["bondType"].size) // 22 % 2).astype(np.int32)
+        if erf:
+            c["potentials"] = c["potentials"] + [dict(kind="erf2", maskI=1, maskJ=2, A=0.3, sigma=0.4, Rp=0.6)]
+        cfgs.append(c)
+    bonds = dict(k=[1.5, 2.5], r0=[0.0, 0.3] if style == 0 else [9.0, 10.0], style=[0, style])
+    alone, grouped = ([engine(c, "GJF", bonds) for c in cfgs] for _ in range(2))
+    grp = gpu.TildGroup(grouped)
+    for n in (1, 4):
+        for e in alone:
+            e.step(n)
+        grp.step(n)
+        for a, b in zip(alone, grouped):
+            for u, v in zip(state(a), state(b)):
+                assert np.isfinite(u).all() and np.array_equal(u, v), n
+    grp.close()
+    for e in alone + grouped:
+        e.close()
