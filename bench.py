@@ -198,10 +198,9 @@ def fts_measure(iters_plain=2000, iters_probe=20, iters_batch=1000, nrep=256, se
 
 def tild_c1_measure(steps=200, replicas=16, seed=1234):
     """The plain TILD diblock melt (2000 chains of 10 A + 10 B, 40 000
-    particles, 20^3 box, 32^3 grid, GJF): stepped alone, as a one-replica
-    graph group (two steps per graph launch), and as a group of `replicas`
-    such systems (different seeds) advanced together; particle-steps/s
-    over all replicas."""
+    particles, 20^3 box, 32^3 grid, GJF): stepped alone, as a group of one,
+    and as a group of `replicas` such systems (different seeds), which share
+    every launch; particle-steps/s over all replicas."""
     import mft
     from mft import systems
     out = {}
@@ -222,12 +221,12 @@ def tild_c1_measure(steps=200, replicas=16, seed=1234):
     eng = systems.tild_engine(cfgs[0], "GJF")
     out["alone"] = timed(eng.step, [eng], 1)
     g1 = mft.TildGroup([eng])
-    out["graph_1"] = timed(g1.step, [eng], 1)
+    out["group_1"] = timed(g1.step, [eng], 1)
     g1.close()
     eng.close()
     engs = [systems.tild_engine(c, "GJF") for c in cfgs]
     g = mft.TildGroup(engs)
-    out[f"graph_{replicas}"] = timed(g.step, engs, replicas)
+    out[f"group_{replicas}"] = timed(g.step, engs, replicas)
     g.close()
     for e in engs:
         e.close()
@@ -354,7 +353,7 @@ def main():
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--no-fts", action="store_true", help="skip the CL-FTS plain/batched measurements")
     ap.add_argument("--no-serve", action="store_true", help="skip the served mixed workload")
-    ap.add_argument("--no-c1", action="store_true", help="skip the 40k-particle diblock (alone, graph, replicas)")
+    ap.add_argument("--no-c1", action="store_true", help="skip the 40k-particle diblock (alone, groups of 1 and 16)")
     ap.add_argument("--serve-window", type=float, default=1.0, help="seconds of Poisson arrivals to serve")
     ap.add_argument("--calibrate-copy", type=int, default=0, metavar="BYTES",
                     help="only run 5 device-to-device copies of BYTES (the known-size kernel that scales the "

@@ -1345,8 +1345,9 @@ static int group_setup(FtsBatch* b, FtsGroup& G)
     G.maxN = 0;
     for (int k = 0; k < nr; ++k)
         for (int m = 0; m < b->reps[G.reps[k]].d.nmolecules; ++m) G.maxN = std::max(G.maxN, b->reps[G.reps[k]].Ntot[m]);
-    // chunks: a replica's per-bead working set is four slices per chain
-    // (q_(s-1) read, the intermediate written and read, e^-W read, q_s written)
+    // chunks: a replica's per-bead working set counts as four slices per chain, those
+    // of the plane and z kernels (q_(s-1) read, the intermediate written and read, e^-W
+    // read, q_s written); the bead kernel has three (its intermediate stays in place)
     std::vector<int> chunk_end;
     size_t acc = 0;
     for (int k = 0; k < nr; ++k) {

@@ -12,8 +12,8 @@
 // instead of two, and per bead a slice of t read and written, E read and q_s
 // written (the two-pass form read q, wrote and read the intermediate, and read
 // E and wrote q: five slices).  Per bead of two chains, against the plane and z
-// kernels before: 32^3 5.5 + 4.6 -> 3.5 us (a dependent launch alone takes 2.7),
-// 64^3 9.0 + 5.1 -> 7.9 us, 96^3 22.2 + 18.9 -> 18.6 us; for three 64^3 replicas
+// kernels before: 32^3 5.5 + 4.6 -> 3.7 us (a dependent launch alone takes 2.7),
+// 64^3 9.0 + 5.1 -> 7.9 us, 96^3 22.2 + 18.9 -> 18.8 us; for three 64^3 replicas
 // 13.1 + 7.7 -> 12.2 us, of which 10.9 are the four slices (4.6 TB/s).
 //
 // Along an axis of N points D is applied as a matrix product, not through the
@@ -301,7 +301,7 @@ __global__ void __launch_bounds__((64 * BeadShape<NX, NA>::W))
                     const float o = bead_swap(d[f][j]), g = bead_swap(e[f][j]);
                     d[f][j] = fmaf(d[f][j], c ? g : e[f][j], o * (c ? e[f][j] : -g));
                     // read again only by the density pass: not kept in the caches
-                    // beside t and E (two 64^3 chains 7.9 -> 7.6 us)
+                    // beside t and E (two 64^3 chains 3 to 4 % faster)
                     if (ok) __builtin_nontemporal_store(d[f][j], (BeadGlobal float*)at(D.q, f, j));
                 }
             }

@@ -784,11 +784,11 @@ def test_three_bond_slots_match_oracle(gpu):
 
 @pytest.mark.parametrize("integrator", ["GJF", "EM"])
 def test_replica_group_graph_equals_engines_alone(gpu, integrator):
-    """Replicas advanced by the group's HIP graph (eight steps of every engine
-    per replay) give the same bits as the same engines stepped alone: three
-    uneven systems, 1 + 17 + 3 + 16 steps (ordinary steps where a replay does
-    not fit, several replays with ordinary steps and host reads between
-    them), every replica checked after each call."""
+    """Replicas of a group whose engines all differ, so that none shares its
+    launches with another and each steps on its own stream, give the same bits
+    as the same engines stepped alone: three uneven systems, 1 + 17 + 3 + 16
+    steps with host reads between them, every replica checked after each call
+    (shared launches: test_gpu_replicas.py)."""
     say("case: replica group", integrator)
     cfgs = [small_system(True, seed=51), small_system(False, seed=52), mixed_charge_system()]
     alone = [systems.tild_engine(c, integrator) for c in cfgs]
