@@ -190,10 +190,6 @@ MFT_PLAN(256, 32, 8, 8, 4)
 // in registers at once (the fused k-space pass): more threads per line,
 // fewer registers per thread, one more LDS pass.  Sizes without one use the
 // default plan.
-// At 20 and 96 points the odd radix and a factor of two are one level: with levels of
-// radix 2 before the odd one the engine's grid forces erred by 12 % more at 96 points
-// than with the default plans, with these by as much (given the densities, 2.22e-7;
-// 2.49e-7; 2.22e-7).
 template <int N>
 struct FftPlanLow : FftPlan<N> {};
 #define MFT_PLAN_LOW(N_, T_, ...)                                               \
@@ -205,14 +201,14 @@ struct FftPlanLow : FftPlan<N> {};
         using R = Radices<__VA_ARGS__>;                                         \
     };
 MFT_PLAN_LOW(16, 4, 4, 4)
-MFT_PLAN_LOW(20, 2, 2, 10)
+MFT_PLAN_LOW(20, 2, 2, 2, 5)
 MFT_PLAN_LOW(24, 4, 2, 2, 2, 3)
 MFT_PLAN_LOW(32, 8, 4, 4, 2)
 MFT_PLAN_LOW(40, 4, 2, 2, 2, 5)
 MFT_PLAN_LOW(48, 8, 2, 2, 2, 2, 3)
 MFT_PLAN_LOW(64, 16, 4, 4, 4)
 MFT_PLAN_LOW(80, 8, 2, 2, 2, 2, 5)
-MFT_PLAN_LOW(96, 16, 2, 2, 2, 2, 6)
+MFT_PLAN_LOW(96, 16, 2, 2, 2, 2, 2, 3)
 MFT_PLAN_LOW(128, 32, 4, 4, 4, 2)
 MFT_PLAN_LOW(160, 16, 2, 2, 2, 2, 2, 5)
 MFT_PLAN_LOW(256, 64, 4, 4, 4, 4)
