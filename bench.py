@@ -55,7 +55,7 @@ def cpu_baseline(seed):
     iterations of the plain 64^3, 100-bead diblock at full size."""
     sys.path.insert(0, os.path.join(ROOT, "oracle"))
     import numpy as np
-    import orc  # the checker; only this leg of the benchmark loads it
+    import orc  # the oracle; only this leg of the benchmark loads it
     from mft import systems
     cores, model = host_info()
     legs = []
